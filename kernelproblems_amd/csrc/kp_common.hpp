@@ -73,6 +73,17 @@ __device__ __forceinline__ void st16(void* p, const u32x4& v) { *reinterpret_cas
 __device__ __forceinline__ void st16_stream(void* p, const u32x4& v) {
   __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
 }
+// The same for rows at any 2-byte address (odd row widths): gfx950 splits a
+// 16-byte access that is not 16-byte aligned itself, so a wave still moves
+// 1 KiB per instruction, over one cache line more.
+typedef uint32_t u32x4_u __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ u32x4 ld16u(const uint16_t* p) { return *reinterpret_cast<const u32x4_u*>(p); }
+__device__ __forceinline__ u32x4 ld16u_stream(const uint16_t* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4_u*>(p));
+}
+__device__ __forceinline__ void st16u_stream(uint16_t* p, const u32x4& v) {
+  __builtin_nontemporal_store(v, reinterpret_cast<u32x4_u*>(p));
+}
 __device__ __forceinline__ void st16f_stream(void* p, const f32x4& v) {
   __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(p));
 }
@@ -117,6 +128,20 @@ __device__ __forceinline__ float wave_sum(float v) {
   return (r0 + r1) + (r2 + r3);
 }
 
+
+// The same within aligned groups of L lanes (8, 16, 32 or the whole wave),
+// every lane of a group ending with its group's sum.
+template <int L>
+__device__ __forceinline__ float lanes_sum(float v) {
+  static_assert(L == 8 || L == 16 || L == 32 || L == 64, "");
+  if constexpr (L == 64) return wave_sum(v);
+  v += dpp_f<0xB1>(v);
+  v += dpp_f<0x4E>(v);
+  v += dpp_f<0x141>(v);
+  if constexpr (L >= 16) v += dpp_f<0x140>(v);
+  if constexpr (L == 32) v += __shfl_xor(v, 16, 64);
+  return v;
+}
 
 __host__ __device__ __forceinline__ int64_t ceil_div_dev(int64_t a, int64_t b) { return (a + b - 1) / b; }
 

@@ -6,6 +6,7 @@
 #include <mutex>
 
 #include "kp_internal.hpp"
+#include "kp_rms_any.hpp"
 #include "kp_rmsnorm_kernels.hpp"
 
 namespace kp {
@@ -328,8 +329,8 @@ size_t fwd_bwd_workspace_size(int64_t M, int64_t N) {
 // Launch plan of a backward row pass: the kernel and its block count (each
 // block writes one weight-gradient partial row).
 struct BwdPlan {
-  BwdKernel vec;   // vectorized kernel, or nullptr for rms_bwd_generic
-  int wpr;         // waves per row of the vectorized kernel
+  BwdKernel vec;   // vectorized kernel (N = 512 * k, 16-byte rows), or nullptr
+  BwdKernel any;   // else the kernel for any width and alignment, or nullptr for rms_bwd_generic
   int threads;     // threads per block
   int blocks;      // row blocks = partial rows
   size_t lds;      // dynamic LDS of the vectorized kernel
@@ -339,7 +340,7 @@ BwdPlan plan_bwd(const void* const* dy_terms, const int64_t* dy_strides, int n_d
                  const int64_t* x_strides, int n_x, const void* weight, int64_t w_seg_len, int64_t w_seg_stride,
                  const void* dx_residual, int64_t dxr_stride, const void* dx, int64_t dx_stride, bool want_dw,
                  const FwdOut* fo, int64_t M, int64_t N) {
-  BwdPlan p{nullptr, 1, kThreads, 0, 0};
+  BwdPlan p{nullptr, nullptr, kThreads, 0, 0};
   if (M <= 0) return p;
   int vpl = 0, wpr = 0, nw = kThreads / 64;
   bool vec = pick_bwd(N, &vpl, &wpr, &nw) && rows_vec_ok(x_terms, x_strides, n_x) &&
@@ -351,10 +352,19 @@ BwdPlan plan_bwd(const void* const* dy_terms, const int64_t* dy_strides, int n_d
   p.vec = vec ? bwd_kernel(vpl, wpr, n_x, n_dy, dx_residual != nullptr, fo != nullptr) : nullptr;
   if (p.vec != nullptr) {
     const int rb = nw / wpr;
-    p.wpr = wpr;
     p.threads = nw * 64;
     p.blocks = bwd_blocks(M, rb, bwd_bpc(nw, (int64_t)(n_x + n_dy + (dx_residual ? 1 : 0)) * vpl * 1024));
     p.lds = (want_dw && rb >= 2) ? (size_t)(rb / 2) * wpr * 512 * vpl * sizeof(float) : 0;
+    return p;
+  }
+  AnyShape as{};
+  if (fo == nullptr && any_bwd_shape(N, &as)) p.any = bwd_any_kernel(as, n_x, n_dy, dx_residual != nullptr);
+  if (p.any != nullptr) {
+    p.threads = kAnyWaves * 64;
+    // at most 2 blocks per CU, as the generic kernel: the partial rows need no
+    // more of a caller's or the static scratch than they did there
+    const int64_t slot = (int64_t)(n_x + n_dy + (dx_residual ? 1 : 0)) * as.vpl * 1024;
+    p.blocks = bwd_blocks(M, kAnyWaves / as.wpr * (64 / as.lpr), auto_bpc(kAnyWaves, slot, 64 * 1024, 2));
   } else {
     p.blocks = bwd_blocks(M, 1, 2);  // generic kernel: one row per block step, 2 blocks per CU
   }
@@ -452,6 +462,9 @@ int rms_bwd_impl(const char* who, const void* const* dy_terms, const int64_t* dy
       void* args[] = {&a};
       launch_dominant_raw(reinterpret_cast<const void*>(plan.vec), dim3(plan.blocks), dim3(plan.threads), args,
                           plan.lds, s);
+    } else if (plan.any != nullptr) {
+      void* args[] = {&a};
+      launch_dominant_raw(reinterpret_cast<const void*>(plan.any), dim3(plan.blocks), dim3(plan.threads), args, 0, s);
     } else {
       KP_LAUNCH_DOMINANT(rms_bwd_generic, dim3(plan.blocks), dim3(kThreads), 0, s, a);
     }
@@ -584,6 +597,14 @@ int kp_rmsnorm_fwd_bf16(const void* const* x_terms, const int64_t* x_strides, in
     const int grid = (int)(groups < cap ? groups : cap);
     void* args[] = {&a};
     launch_dominant_raw(reinterpret_cast<const void*>(fk), dim3(grid), dim3(kThreads), args, 0, s);
+    return check_launch(who);
+  }
+  AnyShape as{};
+  const FwdKernel ak = any_fwd_shape(N, &as) ? fwd_any_kernel(as, n_x) : nullptr;
+  const int64_t groups = ak != nullptr ? ceil_div(M, (int64_t)(4 / as.wpr) * (64 / as.lpr) * as.u) : 0;
+  if (ak != nullptr && groups <= INT32_MAX) {
+    void* args[] = {&a};
+    launch_dominant_raw(reinterpret_cast<const void*>(ak), dim3((unsigned)groups), dim3(kThreads), args, 0, s);
   } else {
     const int64_t cap = (int64_t)cu_count() * 8;
     const int grid = (int)(M < cap ? M : cap);
