@@ -106,8 +106,15 @@ __device__ __forceinline__ FwdTarget row_target(const FwdArgs& a, int64_t row) {
   return FwdTarget{t, a.logits[row * a.rs + (in ? t : 0)]};
 }
 
-// Row-wave epilogue: reduce the lanes' states, then lane 0 writes the row's loss.
-__device__ __forceinline__ void finish_row(const FwdArgs& a, int64_t row, FwdTarget rt, float R, float s) {
+// The states of the NT threads that share a row combined, identical in every
+// one of them: lanes fold by DPP and readlane; the waves' states go through
+// LDS (2 x NT / 64 floats), where the lanes of each wave fold them by DPP
+// again, every 16-lane row the same (folding them one after another took each
+// thread 15 steps of two exponentials a row at NT = 1024).
+template <int NT>
+__device__ __forceinline__ void row_combine(float& R, float& s, float* lds) {
+  constexpr int W = NT / kWave;
+  static_assert(W == 1 || W == 4 || W == 8 || W == 16, "");
   combine_dpp<0xB1>(R, s);   // quad_perm [1,0,3,2]
   combine_dpp<0x4E>(R, s);   // quad_perm [2,3,0,1]
   combine_dpp<0x141>(R, s);  // row_half_mirror
@@ -117,8 +124,27 @@ __device__ __forceinline__ void finish_row(const FwdArgs& a, int64_t row, FwdTar
   float r1 = readlane_f(R, 32), s1 = readlane_f(s, 32);
   combine(r1, s1, readlane_f(R, 48), readlane_f(s, 48));
   combine(r0, s0, r1, s1);
-  if ((threadIdx.x & (kWave - 1)) != 0) return;
-  const double lse = ((double)r0 + log2((double)s0)) / (double)kLog2e;
+  R = r0;
+  s = s0;
+  if constexpr (W > 1) {
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & (kWave - 1);
+    if (lane == 0) {
+      lds[w] = R;
+      lds[W + w] = s;
+    }
+    __syncthreads();
+    R = lds[lane % W];
+    s = lds[W + lane % W];
+    combine_dpp<0xB1>(R, s);
+    combine_dpp<0x4E>(R, s);
+    if constexpr (W > 4) combine_dpp<0x141>(R, s);
+    if constexpr (W > 8) combine_dpp<0x140>(R, s);
+  }
+}
+
+// Row epilogue, by one lane: the row's loss from its combined state.
+__device__ __forceinline__ void finish_row(const FwdArgs& a, int64_t row, FwdTarget rt, float R, float s) {
+  const double lse = ((double)R + log2((double)s)) / (double)kLog2e;
   if (a.lse_out) a.lse_out[row] = (float)lse;
   const int64_t t = rt.t;
   int valid = t != a.ignore;
@@ -141,23 +167,28 @@ constexpr float kStepMax = 0x1p64f;  // a step's sum of 2^(x log2 e - R) above t
 // lane redoes the step exactly with online8, which moves R to the running
 // max.  A stale (smaller) R only scales the lane's sum, which the (R, s)
 // combines take into account.
-template <bool TAIL>
-__device__ __forceinline__ void fwd_step(const u32x4* p, int64_t c0, int64_t cpr, int lane, float& R, float& s) {
+//
+// TAIL: the chunk that crosses the row's end is read as the row's last 8
+// elements (V >= 8), and what the chunk before it holds of them, like every
+// chunk past the end, counts as -inf.
+template <int NT, bool TAIL>
+__device__ __forceinline__ void fwd_step(const uint16_t* p, int64_t c0, int64_t V, int tid, float& R, float& s) {
   u32x4 v[kUnroll];
-  bool ok[kUnroll];
+  int skip[kUnroll];
 #pragma unroll
   for (int u = 0; u < kUnroll; ++u) {
-    const int64_t c = c0 + u * kWave + lane;
-    ok[u] = !TAIL || c < cpr;
-    v[u] = ld16_stream(p + (ok[u] ? c : 0));
+    const int64_t j = (c0 + u * NT + tid) * 8;
+    const int64_t start = !TAIL || j < V - 8 ? j : V - 8;
+    skip[u] = !TAIL ? 0 : j < V ? (int)(j - start) : 8;
+    v[u] = ld16u_stream(p + start);
   }
   float f[kUnroll][8];
 #pragma unroll
   for (int u = 0; u < kUnroll; ++u) {
     unpack8(v[u], f[u]);
-    if (TAIL && !ok[u]) {
+    if (TAIL) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) f[u][i] = -INFINITY;
+      for (int i = 0; i < 8; ++i) f[u][i] = i < skip[u] ? -INFINITY : f[u][i];
     }
   }
   float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -174,71 +205,92 @@ __device__ __forceinline__ void fwd_step(const u32x4* p, int64_t c0, int64_t cpr
   }
 }
 
-// One wave per row, rows 16-byte granular (V % 8 == 0, aligned): lane l reads
-// chunks (k * 64 + l), k = 0, 1, ... of the row, kUnroll per step, all loads
-// of a step issued together.  Full steps carry no masks; the tail step's
-// chunks past the row end read the row's first chunk and count as -inf.
-__global__ __launch_bounds__(kThreads) void xent_fwd_vec(FwdArgs a) {
-  const int64_t row = (int64_t)blockIdx.x * kWavesPerBlock + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+// NT threads per row (64: a wave, four rows a block; else a block per row),
+// any stride and alignment, V >= 8: thread t reads chunks (k * NT + t) of 8
+// elements, kUnroll per step, all loads of a step issued together.  Only the
+// last step carries masks.
+template <int NT>
+__global__ __launch_bounds__(NT < kThreads ? kThreads : NT) void xent_fwd_vec(FwdArgs a) {
+  __shared__ float red[2 * NT / kWave];
+  const int64_t row = NT == kWave ? (int64_t)blockIdx.x * kWavesPerBlock +
+                                        __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))
+                                  : (int64_t)blockIdx.x;
   if (row >= a.M) return;
   const FwdTarget rt = row_target(a, row);
-  const int lane = threadIdx.x & (kWave - 1);
-  const u32x4* p = reinterpret_cast<const u32x4*>(a.logits + row * a.rs);
-  const int64_t cpr = a.V / 8;
-  constexpr int64_t kStep = (int64_t)kUnroll * kWave;
-  const int64_t full = cpr / kStep * kStep;
+  const int tid = NT == kWave ? threadIdx.x & (kWave - 1) : threadIdx.x;
+  const uint16_t* p = a.logits + row * a.rs;
+  constexpr int64_t kStep = (int64_t)kUnroll * NT;
+  const int64_t full = a.V / 8 / kStep * kStep;
   float R = -INFINITY, s = 0.0f;
-  for (int64_t c0 = 0; c0 < full; c0 += kStep) fwd_step<false>(p, c0, cpr, lane, R, s);
-  if (full < cpr) fwd_step<true>(p, full, cpr, lane, R, s);
-  finish_row(a, row, rt, R, s);
+  for (int64_t c0 = 0; c0 < full; c0 += kStep) fwd_step<NT, false>(p, c0, a.V, tid, R, s);
+  if (full * 8 < a.V) fwd_step<NT, true>(p, full, a.V, tid, R, s);
+  row_combine<NT>(R, s, red);
+  if (tid == 0) finish_row(a, row, rt, R, s);
 }
 
-// Any row stride / alignment / V: lane l reads elements l, l + 64, ...
+// V < 8: lane l holds element l.
 __global__ __launch_bounds__(kThreads) void xent_fwd_scalar(FwdArgs a) {
   const int64_t row = (int64_t)blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
   if (row >= a.M) return;
   const FwdTarget rt = row_target(a, row);
   const int lane = threadIdx.x & (kWave - 1);
-  const uint16_t* p = a.logits + row * a.rs;
+  float f[8] = {lane < a.V ? bf_to_f(a.logits[row * a.rs + lane]) : -INFINITY,
+                -INFINITY, -INFINITY, -INFINITY, -INFINITY, -INFINITY, -INFINITY, -INFINITY};
   float R = -INFINITY, s = 0.0f;
-  for (int64_t j0 = 0; j0 < a.V; j0 += 8 * kWave) {
-    float f[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int64_t j = j0 + i * kWave + lane;
-      f[i] = j < a.V ? bf_to_f(p[j]) : -INFINITY;
-    }
-    online8(R, s, f);
-  }
-  finish_row(a, row, rt, R, s);
+  online8(R, s, f);
+  row_combine<kWave>(R, s, nullptr);
+  if (lane == 0) finish_row(a, row, rt, R, s);
 }
 
 // One block: loss = scale * sum(row_loss), total_weight = sum(row_valid), in a
-// fixed order (thread t sums rows t, t + 1024, ... in fp64, then a tree).
+// fixed order: thread t sums rows t, t + 1024, ... in fp64 (four of them
+// requested together), lanes fold by shuffles, then the first wave folds the
+// 16 wave sums (one barrier; a tree through LDS with a barrier per level
+// made this launch 4.2 us).
 constexpr int kFinThreads = 1024;
+__device__ __forceinline__ double wave_sum_f64(double v) {
+#pragma unroll
+  for (int m = 1; m < kWave; m <<= 1) v += __shfl_xor(v, m, kWave);
+  return v;
+}
 __global__ __launch_bounds__(kFinThreads) void xent_fwd_finish(const double* row_loss, const int32_t* row_valid,
                                                                 int64_t M, double scale, float* loss, float* total_weight) {
-  __shared__ double ls[kFinThreads];
-  __shared__ int64_t cs[kFinThreads];
-  double acc = 0.0;
-  int64_t cnt = 0;
-  for (int64_t i = threadIdx.x; i < M; i += kFinThreads) {
-    acc += row_loss[i];
-    cnt += row_valid[i];
-  }
-  ls[threadIdx.x] = acc;
-  cs[threadIdx.x] = cnt;
-  __syncthreads();
-  for (int w = kFinThreads / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) {
-      ls[threadIdx.x] += ls[threadIdx.x + w];
-      cs[threadIdx.x] += cs[threadIdx.x + w];
+  constexpr int kW = kFinThreads / kWave;
+  __shared__ double ls[kW], cs[kW];
+  double acc = 0.0, cnt = 0.0;  // counts below 2^53 are exact in any order
+  int64_t i = threadIdx.x;
+  for (; i + 3 * kFinThreads < M; i += 4 * kFinThreads) {
+    double l[4];
+    int32_t c[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      l[k] = row_loss[i + k * kFinThreads];
+      c[k] = row_valid[i + k * kFinThreads];
     }
-    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      acc += l[k];
+      cnt += (double)c[k];
+    }
   }
-  if (threadIdx.x == 0) {
-    loss[0] = (float)(ls[0] * scale);
-    total_weight[0] = (float)cs[0];
+  for (; i < M; i += kFinThreads) {
+    acc += row_loss[i];
+    cnt += (double)row_valid[i];
+  }
+  acc = wave_sum_f64(acc);
+  cnt = wave_sum_f64(cnt);
+  const int lane = threadIdx.x & (kWave - 1);
+  if (lane == 0) {
+    ls[threadIdx.x >> 6] = acc;
+    cs[threadIdx.x >> 6] = cnt;
+  }
+  __syncthreads();
+  if (threadIdx.x >= kWave) return;
+  acc = wave_sum_f64(lane < kW ? ls[lane] : 0.0);
+  cnt = wave_sum_f64(lane < kW ? cs[lane] : 0.0);
+  if (lane == 0) {
+    loss[0] = (float)(acc * scale);
+    total_weight[0] = (float)cnt;
   }
 }
 
@@ -335,13 +387,14 @@ __global__ __launch_bounds__(kThreads) void xent_bwd_scalar(BwdArgs a) {
 // logits (the _log_softmax -> nll_loss_forward -> nll_loss_backward ->
 // _log_softmax_backward_data region with the fp32 log-softmax never stored),
 // optionally with the forward's loss.  A row needs its lse before its first
-// gradient, so a whole row is held on chip: one 1024-thread block per row,
-// thread t holding chunks t + 1024 k (k < KC) in registers -- 16 chunks
-// (64 VGPRs) cover V <= 131072, e.g. the 128256-entry vocabulary (256 KB of
+// gradient, so a whole row is held on chip: NT threads per row, thread t
+// holding chunks t + NT k (k < KC) in registers -- 16 chunks (64 VGPRs) of
+// 1024 threads cover V <= 131072, e.g. the 128256-entry vocabulary (256 KB of
 // bf16 per row).  Each element is read once and written once: 4 bytes per
 // element instead of the 6 of a forward pass followed by a pass that re-reads
 // the logits.  The lse comes from the same (R, s) states as the forward
-// (exponents by one fma against R = fl(max L)), combined across the block.
+// (exponents by one fma against R = fl(max L)), combined across the row's
+// threads.
 struct FbArgs {
   const uint16_t* logits;
   int64_t rs;  // row stride, elements
@@ -357,70 +410,63 @@ struct FbArgs {
   int32_t* err;
 };
 
-constexpr int kFbThreads = 1024;
-constexpr int kFbMaxChunks = 16;  // 16-byte chunks per thread held in registers
-
-// The row's combined (R, s), identical in every thread of the block: lanes
-// fold by DPP and readlane, waves through LDS in a fixed order.
-template <int NWAVES>
-__device__ __forceinline__ void block_combine(float& R, float& s, float* lds) {
-  combine_dpp<0xB1>(R, s);
-  combine_dpp<0x4E>(R, s);
-  combine_dpp<0x141>(R, s);
-  combine_dpp<0x140>(R, s);
-  float r0 = readlane_f(R, 0), s0 = readlane_f(s, 0);
-  combine(r0, s0, readlane_f(R, 16), readlane_f(s, 16));
-  float r1 = readlane_f(R, 32), s1 = readlane_f(s, 32);
-  combine(r1, s1, readlane_f(R, 48), readlane_f(s, 48));
-  combine(r0, s0, r1, s1);
-  const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & (kWave - 1)) == 0) {
-    lds[w] = r0;
-    lds[NWAVES + w] = s0;
-  }
-  __syncthreads();
-  R = lds[0];
-  s = lds[NWAVES];
-#pragma unroll
-  for (int i = 1; i < NWAVES; ++i) combine(R, s, lds[i], lds[NWAVES + i]);
-}
-
 struct RowTarget {
-  int64_t t;     // target column, -1 when the row has none
-  float sum;     // s_i = sum_j grad_ij: -g, or 0
+  int64_t t;  // target column, -1 when the row has none
   bool valid;
 };
 
-__device__ __forceinline__ RowTarget fb_target_of(const FbArgs& a, int64_t t) {
+__device__ __forceinline__ RowTarget fb_target_of(const FbArgs& a, int64_t t, int tid) {
   const bool in_range = t >= 0 && t < a.V;
   const bool valid = t != a.ignore && in_range;
-  if (t != a.ignore && !in_range && threadIdx.x == 0 && a.err) a.err[0] = 1;
-  return RowTarget{valid ? t : -1, valid ? -a.g : 0.0f, valid};
-}
-__device__ __forceinline__ RowTarget fb_target(const FbArgs& a, int64_t row) {
-  return fb_target_of(a, target_at(a.targets, a.tbytes, row));
+  if (t != a.ignore && !in_range && tid == 0 && a.err) a.err[0] = 1;
+  return RowTarget{valid ? t : -1, valid};
 }
 
-// Thread 0 records the row's loss lse - x_t (x_t loaded before any store of
-// the row, so out may alias the logits).  lse = (R + log2 s) / L with the
-// fp32 log2 s of the gradient (|log2 s| < 18 for V < 2^17: within 2^-24 x 18
-// of exact), summed and divided in fp64.
-__device__ __forceinline__ void fb_row_loss(const FbArgs& a, int64_t row, const RowTarget& rt, float R, float lg,
+// One lane records the row's loss lse - x_t (x_t loaded before any store of
+// the row, so out may alias the logits).  lse = (R + log2 s) / L with fp32
+// log2 s (|log2 s| < 18 for V < 2^17: within 2^-24 x 18 of exact), summed and
+// divided in fp64.
+__device__ __forceinline__ void fb_row_loss(const FbArgs& a, int64_t row, const RowTarget& rt, float R, float s,
                                             float xt) {
-  if (a.row_loss == nullptr || threadIdx.x != 0) return;
-  const double lse = ((double)R + (double)lg) / (double)kLog2e;
+  const double lse = ((double)R + (double)log2f(s)) / (double)kLog2e;
   a.row_loss[row] = rt.valid ? lse - (double)xt : 0.0;
   a.row_valid[row] = rt.valid;
 }
 
-// p = exp(x - lse) = 2^((x L - R) - log2 s): the fma is rounded relative to
-// x L - R (small for the large p), and log2 s is subtracted afterwards, so
-// p near 1 (a confident row's target, where grad - p sum cancels) carries
-// fp32 relative error rather than an absolute error of ulp(R).
-__device__ __forceinline__ float fb_grad(float x, float R, float lg, bool is_target, float g, float sum) {
-  const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(x, kLog2e, -R) - lg);
-  const float grad = is_target ? -g : 0.0f;
-  return grad - p * sum;
+// p g = exp(x - lse) g = 2^(x L - R) (g / s): the fma is rounded relative to
+// x L - R (small for the large p), and k = g / s carries fp32 relative error.
+// The target's entry is (p - 1) g with p = exp / s divided out first: p near 1
+// (a confident row) has fp32 relative error, and p = 1 gives exactly 0.  A row
+// without a target has k = 0.
+__device__ __forceinline__ float fb_exp(float x, float R) {
+  return __builtin_amdgcn_exp2f(__builtin_fmaf(x, kLog2e, -R));
+}
+
+__device__ __forceinline__ float fb_target_grad(float xt, float R, float s, float g) {
+  return __builtin_fmaf(fb_exp(xt, R) / s, g, -g);
+}
+
+// Max of the bf16 values of KC packed chunks, as fp32.  bf16 values order as
+// signed 16-bit integers while one of them is not negative: one packed max
+// per two values instead of two unpacks and a max.  All negative: their order
+// is that of unsigned integers reversed.
+template <int KC>
+__device__ __forceinline__ float packed_max(const u32x4* v) {
+  typedef int16_t s16x2 __attribute__((ext_vector_type(2)));
+  typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+  s16x2 m = {INT16_MIN, INT16_MIN};
+#pragma unroll
+  for (int k = 0; k < KC; ++k)
+#pragma unroll
+    for (int d = 0; d < 4; ++d) m = __builtin_elementwise_max(m, __builtin_bit_cast(s16x2, (uint32_t)v[k][d]));
+  const int16_t top = m[0] > m[1] ? m[0] : m[1];
+  if (top >= 0) return bf_to_f((uint16_t)top);
+  u16x2 n = {0xffff, 0xffff};
+#pragma unroll
+  for (int k = 0; k < KC; ++k)
+#pragma unroll
+    for (int d = 0; d < 4; ++d) n = __builtin_elementwise_min(n, __builtin_bit_cast(u16x2, (uint32_t)v[k][d]));
+  return bf_to_f(n[0] < n[1] ? n[0] : n[1]);
 }
 
 // An empty asm that takes the packed chunks as in/out operands: the values
@@ -433,33 +479,11 @@ __device__ __forceinline__ void keep_packed(u32x4* v) {
   for (int k = 0; k < KC; ++k) asm volatile("" : "+v"(v[k]));
 }
 
-// Rows are addressed through raw buffer descriptors: the row base and length
-// sit in SGPRs and each access takes a single 32-bit offset VGPR, where a
-// 64-bit address takes two (32 per row at KC = 16, which spill).  The range
-// check of the descriptor covers the VGPR offset: a load past the row end
-// returns zeros and a store past it is dropped, so chunks beyond the row get
-// the offset 0x80000000 (out of range for any row) instead of a branch, and
-// a descriptor of length 0 fetches nothing.  Word 3 0x00020000 is the
-// raw-buffer setting of the gfx9 family (32-bit data format).
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
-constexpr int kBufNT = 2;               // cache policy: non-temporal
-constexpr uint32_t kOutOfRange = 0x80000000u;
-
+// Word 3 0x00020000 is the raw-buffer setting of the gfx9 family (32-bit data
+// format); loads past `bytes` return zeros.
 __device__ __forceinline__ rsrc_t row_rsrc(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
-}
-
-// Byte offset of chunk k of thread tid, or kOutOfRange past the row.
-__device__ __forceinline__ uint32_t fb_off(int tid, int k, int64_t cpr) {
-  const int64_t c = tid + (int64_t)k * kFbThreads;
-  return c < cpr ? (uint32_t)c * 16u : kOutOfRange;
-}
-
-// All KC loads of a row, issued together.
-template <int KC>
-__device__ __forceinline__ void fb_load_row(rsrc_t r, int tid, int64_t cpr, u32x4* v) {
-#pragma unroll
-  for (int k = 0; k < KC; ++k) v[k] = __builtin_amdgcn_raw_buffer_load_b128(r, fb_off(tid, k, cpr), 0, kBufNT);
 }
 
 // Target of `row` (int32 or int64 ids) by two 4-byte buffer loads and no
@@ -481,98 +505,157 @@ __device__ __forceinline__ int64_t fb_target_value(const FbArgs& a, uint32_t lo,
   return a.tbytes == 8 ? (int64_t)(((uint64_t)hi << 32) | lo) : (int64_t)(int32_t)lo;
 }
 
-// Persistent: one block per CU walks rows blockIdx.x, + gridDim.x, ...; the
-// next row's loads are issued as soon as the previous row's stores are, so
-// the store stream of one row overlaps the load stream of the next (754 us
-// against 791 us for one fresh block per row at [8192, 128256]).  Issuing
-// the next row's chunk k right after row r's chunk k is unpacked, interleaved
-// with row r's stores, measured slower (808 us).  The LDS slots of the block
-// reduction alternate between rows (a slow wave may still read row r's slots
-// while a fast one writes row r + 1's).
-template <int KC>
-__global__ __launch_bounds__(kFbThreads) void xent_fwd_bwd_vec(FbArgs a) {
-  constexpr int kWaves = kFbThreads / kWave;
-  __shared__ float red[2][2 * kWaves];
-  const int64_t cpr = a.V / 8;
-  const uint32_t row_bytes = (uint32_t)a.V * 2u;
+// Chunks whose exponentials stay in fp32 registers from the sum to the
+// gradient (8 registers in place of 4), as many as 128 VGPRs hold beside the
+// packed ones; the others take theirs a second time.  Rows of several blocks
+// a CU gain by it ([4096, 32000] 92.8 us with one kept, 90.0 us so); one row a
+// CU waits for memory instead (NT = 1024, [8192, 128256]: 740 us with eight
+// kept, 735 us with one).
+constexpr int fb_kept(int nt, int kc) { return nt == 1024 ? 1 : kc < 12 ? kc : kc == 12 ? 11 : 24 - kc; }
+
+// Any stride and alignment (16-byte accesses at 2-byte alignment from a
+// scalar row base and a 32-bit offset), V >= 8, KC = ceil(ceil(V / 8) / NT):
+// chunk k < KC - 1 of every thread lies inside the row.  The chunk that
+// crosses the row's end is read as the row's last 8 elements; those that the
+// chunk before it holds, like whole chunks past the end, are -inf for the max
+// and the sum, and the rest are stored one by one.
+//
+// NT = 1024 (V > 65528) is persistent: one block per CU walks rows
+// blockIdx.x, + gridDim.x, ...; the next row's loads are issued as soon as
+// the previous row's stores are, so the store stream of one row overlaps the
+// load stream of the next (754 us against 791 us for one fresh block per row
+// at [8192, 128256]).  Issuing the next row's chunk k right after row r's
+// chunk k is unpacked, interleaved with row r's stores, measured slower
+// (808 us).  Shorter rows take fewer threads, so that several rows are in
+// different phases on a CU.  The LDS slots of the row reduction alternate
+// between rows (a slow wave may still read row r's slots while a fast one
+// writes row r + 1's).
+//
+// Bound by HBM: a third less VALU work per element (packed maxima, the target
+// and 1 / s out of the gradient's inner loop) only took [8192, 128256] from
+// 752 to 735 us, of 640 us for a plain copy of its bytes -- a row's loads,
+// reduction and stores follow one another on its CU.  Rows that are not
+// 16-byte aligned cost 1.17x ([2048, 50257] 95.5 us, [2048, 50256] 81.7 us;
+// the scalar two-pass kernel they took before 252 us); plain (write-back)
+// stores or loads are slower at either alignment (97.9 and 97.3 us, and
+// 85.4 and 82.5 us).  Threads by the row's length, against one persistent
+// 1024-thread block per CU for every V: [4096, 32000] 123 -> 90 us,
+// [8192, 8192] 142 -> 48 us, [8192, 1003] 28 us (scalar) -> 12.5 us.
+template <int NT, int KC>
+__global__ __launch_bounds__(NT < kThreads ? kThreads : NT, KC > 8 ? 4 : 1) void xent_fwd_bwd_vec(FbArgs a) {
+  constexpr int kRows = NT < kThreads ? kThreads / NT : 1;
+  constexpr int KE = fb_kept(NT, KC);
+  __shared__ float red[2][2 * NT / kWave];
+  const int V = (int)a.V, cpr = (V + 7) / 8;
   u32x4 v[KC];
   int parity = 0;
-  for (int64_t row = blockIdx.x; row < a.M; row += gridDim.x, parity ^= 1) {
+  const int64_t r0 = (int64_t)blockIdx.x * kRows +
+                     (kRows > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0);
+  for (int64_t row = r0; row < a.M; row += (int64_t)gridDim.x * kRows, parity ^= 1) {
     // the thread index passes through an empty asm each row, so the chunk
     // offsets derived from it are recomputed where they are used instead of
     // being hoisted out of the loop (16 more live VGPRs)
-    int tid = threadIdx.x;
+    int tid = kRows > 1 ? threadIdx.x & (kWave - 1) : threadIdx.x;
     asm volatile("" : "+v"(tid));
     // the row's target is requested ahead of its data: vmcnt counts in issue
     // order, so waiting for the target afterwards does not wait for the row
     uint32_t t_lo, t_hi;
     fb_target_load(a, row, t_lo, t_hi);
     __builtin_amdgcn_sched_barrier(0);
-    fb_load_row<KC>(row_rsrc(a.logits + row * a.rs, row_bytes), tid, cpr, v);
+    const char* xr = reinterpret_cast<const char*>(a.logits + row * a.rs);
+    int cl = tid + (KC - 1) * NT;  // the last chunk, where it starts and how much of it is another's
+    int start = cl * 8 < V - 8 ? cl * 8 : V - 8;
+    int skip = cl < cpr ? cl * 8 - start : 8;
+#pragma unroll
+    for (int k = 0; k < KC; ++k)
+      v[k] = ld16u_stream(reinterpret_cast<const uint16_t*>(
+          xr + (k < KC - 1 ? (uint32_t)(tid + k * NT) * 16u : (uint32_t)start * 2u)));
     __builtin_amdgcn_sched_barrier(0);
-    const rsrc_t ro = row_rsrc(a.out + row * a.ors, row_bytes);
-    const RowTarget rt = fb_target_of(a, fb_target_value(a, t_lo, t_hi));
-    // x_t for the row loss, loaded by every lane without a branch (an invalid
-    // target reads out of range: 0) and consumed only before the block
-    // combine, so its wait is not a wait for the whole row; thread 0 uses it
-    uint16_t xtb = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(
-        row_rsrc(a.logits + row * a.rs, row_bytes), rt.valid ? (uint32_t)rt.t * 2u : kOutOfRange, 0, 0);
-    float m = -INFINITY;
+    const RowTarget rt = fb_target_of(a, fb_target_value(a, t_lo, t_hi), tid);
+    // x_t, loaded by every lane without a branch (element 0 where there is no
+    // target) and consumed only before the row reduction, so its wait is not
+    // a wait for the whole row
+    uint16_t xtb = *reinterpret_cast<const uint16_t*>(xr + (uint32_t)(rt.valid ? (int)rt.t : 0) * 2u);
+    if (skip > 0) {
 #pragma unroll
-    for (int k = 0; k < KC; ++k) {
-      if (tid + (int64_t)k * kFbThreads < cpr) {
-        float f[8];
-        unpack8(v[k], f);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) m = fmaxf(m, f[i]);
+      for (int d = 0; d < 4; ++d) {
+        const uint32_t m = (2 * d < skip ? 0xffffu : 0u) | (2 * d + 1 < skip ? 0xffff0000u : 0u);
+        v[KC - 1][d] = (v[KC - 1][d] & ~m) | (0xff80ff80u & m);
       }
     }
+    float R = packed_max<KC>(v) * kLog2e, s = 0.0f;
     keep_packed<KC>(v);
-    float R = m * kLog2e, s = 0.0f;
-    if (R != -INFINITY) {
+    float e[KE][8];
+    const float Rl = R;
+    {
+      const float ref = R == -INFINITY ? 0.0f : R;  // nothing but -inf: every exponential is 0
       float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int k = 0; k < KC; ++k) {
-        if (tid + (int64_t)k * kFbThreads < cpr) {
-          float f[8];
-          unpack8(v[k], f);
+        float f[8];
+        unpack8(v[k], f);
 #pragma unroll
-          for (int i = 0; i < 8; ++i) part[i & 3] += __builtin_amdgcn_exp2f(__builtin_fmaf(f[i], kLog2e, -R));
+        for (int i = 0; i < 8; ++i) {
+          const float x = fb_exp(f[i], ref);
+          if (k < KE) e[k][i] = x;
+          part[i & 3] += x;
         }
       }
       s = (part[0] + part[1]) + (part[2] + part[3]);
     }
     asm volatile("" : "+v"(xtb));  // x_t has arrived before the barrier: other waves may overwrite it after
-    const float xt = (a.row_loss != nullptr && tid == 0 && rt.valid) ? bf_to_f(xtb) : 0.0f;
-    block_combine<kWaves>(R, s, red[parity]);
-    const float lg = log2f(s);
-    fb_row_loss(a, row, rt, R, lg, xt);
-    keep_packed<KC>(v);
-    const int64_t tc = rt.t >> 3;  // -1 >> 3 = -1: no chunk matches
-    const int ti = (int)(rt.t & 7);
+    const float xt = bf_to_f(xtb);
+    row_combine<NT>(R, s, red[parity]);
+    if (a.row_loss != nullptr && tid == 0) fb_row_loss(a, row, rt, R, s, xt);
+    const float kf = rt.valid ? a.g / s : 0.0f;
+    const float kl = Rl == R ? kf : kf * __builtin_amdgcn_exp2f(Rl - R);  // for the kept exponentials, against Rl
+    keep_packed<KC - KE>(v + KE);
     asm volatile("" : "+v"(tid));  // the store offsets are recomputed here, not kept from the loads
+    char* out = reinterpret_cast<char*>(a.out + row * a.ors);
 #pragma unroll
     for (int k = 0; k < KC; ++k) {
-      const int64_t c = tid + (int64_t)k * kFbThreads;
-      float f[8], o[8];
-      unpack8(v[k], f);
-      const uint32_t off = fb_off(tid, k, cpr);
+      float o[8];
+      if (k < KE) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) o[i] = fb_grad(f[i], R, lg, c == tc && i == ti, a.g, rt.sum);
-      __builtin_amdgcn_raw_buffer_store_b128(pack8(o), ro, off, 0, kBufNT);
+        for (int i = 0; i < 8; ++i) o[i] = e[k][i] * kl;
+      } else {
+        float f[8];
+        unpack8(v[k], f);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[i] = fb_exp(f[i], R) * kf;
+      }
+      if (k < KC - 1) {
+        st16u_stream(reinterpret_cast<uint16_t*>(out + (uint32_t)(tid + k * NT) * 16u), pack8(o));
+      } else {
+        cl = tid + (KC - 1) * NT;
+        start = cl * 8 < V - 8 ? cl * 8 : V - 8;
+        skip = cl < cpr ? cl * 8 - start : 8;
+        uint16_t* q = reinterpret_cast<uint16_t*>(out + (uint32_t)start * 2u);
+        if (skip == 0) {
+          st16u_stream(q, pack8(o));
+        } else {
+#pragma unroll
+          for (int i = 1; i < 8; ++i)
+            if (i >= skip) q[i] = f_to_bf(o[i]);
+        }
+      }
     }
+    // the target's entry once more, by the thread that stored it above
+    if (rt.valid && tid == ((int)rt.t >> 3) % NT)
+      *reinterpret_cast<uint16_t*>(out + (uint32_t)rt.t * 2u) = f_to_bf(fb_target_grad(xt, R, s, a.g));
   }
 }
 
-// Any V, stride or alignment: 256 threads per row, two passes over the row
-// (the second re-reads it); each element is read before it is written by the
-// same thread, so out may alias the logits here too.
+// Rows wider than the register kernel holds (or V < 8): 256 threads per row,
+// two passes over the row (the second re-reads it); each element is read
+// before it is written by the same thread, so out may alias the logits here
+// too.
 __global__ __launch_bounds__(kThreads) void xent_fwd_bwd_scalar(FbArgs a) {
   __shared__ float red[2 * kWavesPerBlock];
   const int64_t row = blockIdx.x;
   const uint16_t* x = a.logits + row * a.rs;
   uint16_t* o = a.out + row * a.ors;
-  const RowTarget rt = fb_target(a, row);
+  const RowTarget rt = fb_target_of(a, target_at(a.targets, a.tbytes, row), threadIdx.x);
   const float xt = (a.row_loss != nullptr && threadIdx.x == 0 && rt.valid) ? bf_to_f(x[rt.t]) : 0.0f;
   float R = -INFINITY, s = 0.0f;
   for (int64_t j0 = 0; j0 < a.V; j0 += 8 * kThreads) {
@@ -585,21 +668,35 @@ __global__ __launch_bounds__(kThreads) void xent_fwd_bwd_scalar(FbArgs a) {
     online8(R, s, f);
   }
   asm volatile("" ::"v"(xt));  // x_t has arrived before the barrier: other waves may overwrite it after
-  block_combine<kWavesPerBlock>(R, s, red);
-  const float lg = log2f(s);
-  fb_row_loss(a, row, rt, R, lg, xt);
-  for (int64_t j = threadIdx.x; j < a.V; j += kThreads)
-    o[j] = f_to_bf(fb_grad(bf_to_f(x[j]), R, lg, j == rt.t, a.g, rt.sum));
+  row_combine<kThreads>(R, s, red);
+  if (a.row_loss != nullptr && threadIdx.x == 0) fb_row_loss(a, row, rt, R, s, xt);
+  const float kf = rt.valid ? a.g / s : 0.0f;
+  for (int64_t j = threadIdx.x; j < a.V; j += kThreads) {
+    const float xj = bf_to_f(x[j]);
+    o[j] = f_to_bf(j == rt.t ? fb_target_grad(xj, R, s, a.g) : fb_exp(xj, R) * kf);
+  }
 }
 
-const void* fwd_bwd_vec_kernel(int kc) {
-  switch (kc) {
-    case 1: return reinterpret_cast<const void*>(xent_fwd_bwd_vec<1>);
-    case 2: return reinterpret_cast<const void*>(xent_fwd_bwd_vec<2>);
-    case 4: return reinterpret_cast<const void*>(xent_fwd_bwd_vec<4>);
-    case 8: return reinterpret_cast<const void*>(xent_fwd_bwd_vec<8>);
-    default: return reinterpret_cast<const void*>(xent_fwd_bwd_vec<16>);
-  }
+// The register kernel for rows of V elements: NT threads per row and KC
+// chunks per thread, or false.
+typedef void (*FbKernel)(FbArgs);
+template <int NT, int KC, int KMAX>
+FbKernel fb_pick(int kc) {
+  if constexpr (KC > KMAX) return nullptr;
+  else return kc == KC ? xent_fwd_bwd_vec<NT, KC> : fb_pick<NT, KC + 1, KMAX>(kc);
+}
+struct FbPlan {
+  FbKernel kernel;
+  int threads, rows;  // per block
+  bool persistent;
+};
+FbPlan fb_plan(int64_t V) {
+  const int64_t cpr = ceil_div(V, 8);
+  if (V < 8 || cpr > 16 * 1024) return FbPlan{nullptr, 0, 0, false};
+  if (cpr <= 512) return FbPlan{fb_pick<64, 1, 8>((int)ceil_div(cpr, 64)), kThreads, kThreads / 64, false};
+  if (cpr <= 2048) return FbPlan{fb_pick<256, 3, 8>((int)ceil_div(cpr, 256)), 256, 1, false};
+  if (cpr <= 8192) return FbPlan{fb_pick<512, 5, 16>((int)ceil_div(cpr, 512)), 512, 1, false};
+  return FbPlan{fb_pick<1024, 9, 16>((int)ceil_div(cpr, 1024)), 1024, 1, true};
 }
 
 bool valid_target_bytes(int b) { return b == 4 || b == 8; }
@@ -645,11 +742,16 @@ int kp_cross_entropy_fwd_bf16(const void* logits, int64_t row_stride, int64_t M,
   a.lse_out = row_lse;
   a.err = error_flag;
   if (M > 0) {
-    const bool vec = V % 8 == 0 && aligned16(logits) && (M == 1 || row_stride % 8 == 0);
-    const unsigned blocks = (unsigned)ceil_div(M, kWavesPerBlock);
+    // Threads per row: a wave while there are rows enough to fill the chip,
+    // then a block (a wave streams a row at a few GB/s by itself).
+    const int nt = V < 8 ? 0 : M >= 2048 || V < 8192 ? 64 : M >= 512 || V < 32768 ? 256 : 1024;
+    const void* fk = nt == 0     ? reinterpret_cast<const void*>(xent_fwd_scalar)
+                     : nt == 64  ? reinterpret_cast<const void*>(xent_fwd_vec<64>)
+                     : nt == 256 ? reinterpret_cast<const void*>(xent_fwd_vec<256>)
+                                 : reinterpret_cast<const void*>(xent_fwd_vec<1024>);
+    const unsigned blocks = (unsigned)(nt > 64 ? M : ceil_div(M, kWavesPerBlock));
     void* args[] = {&a};
-    launch_dominant_raw(reinterpret_cast<const void*>(vec ? xent_fwd_vec : xent_fwd_scalar), dim3(blocks),
-                        dim3(kThreads), args, 0, st);
+    launch_dominant_raw(fk, dim3(blocks), dim3(nt > kThreads ? nt : kThreads), args, 0, st);
     const int rc = check_launch(who);
     if (rc != KP_OK) return rc;
   }
@@ -736,18 +838,13 @@ int kp_cross_entropy_fwd_bwd_bf16(const void* logits, int64_t row_stride, int64_
     a.row_valid = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + (size_t)M * sizeof(double));
   }
   if (M > 0) {
-    const int64_t cpr = V / 8;
-    const bool vec = V % 8 == 0 && aligned16(logits) && aligned16(grad_logits) &&
-                     (M == 1 || (row_stride % 8 == 0 && out_row_stride % 8 == 0)) &&
-                     cpr <= (int64_t)kFbThreads * kFbMaxChunks &&
-                     M * target_bytes <= 0xffffffffLL;  // the targets' buffer descriptor is 32-bit
+    // the targets' buffer descriptor is 32-bit
+    const FbPlan plan = M * target_bytes <= 0xffffffffLL ? fb_plan(V) : FbPlan{nullptr, 0, 0, false};
     void* args[] = {&a};
-    if (vec) {
-      int kc = 1;
-      while ((int64_t)kc * kFbThreads < cpr) kc *= 2;
-      const int64_t cus = cu_count();
-      const unsigned blocks = (unsigned)(M < cus ? M : cus);
-      launch_dominant_raw(fwd_bwd_vec_kernel(kc), dim3(blocks), dim3(kFbThreads), args, 0, st);
+    if (plan.kernel != nullptr) {
+      const int64_t cus = cu_count(), groups = ceil_div(M, plan.rows);
+      const unsigned blocks = (unsigned)(plan.persistent && groups > cus ? cus : groups);
+      launch_dominant_raw(reinterpret_cast<const void*>(plan.kernel), dim3(blocks), dim3(plan.threads), args, 0, st);
     } else {
       launch_dominant_raw(reinterpret_cast<const void*>(xent_fwd_bwd_scalar), dim3((unsigned)M), dim3(kThreads), args,
                           0, st);
