@@ -485,13 +485,13 @@ class SwiGlu(Workload):
 
     # mode -> (inputs, outputs, entry point, dominant kernel, description)
     MODES = {
-        "fwd": (2, 1, "kp_swiglu_fwd_bf16", "swiglu_fwd_vec",
+        "fwd": (2, 1, "kp_swiglu_fwd_bf16", "swiglu_vec",
                 "SwiGLU gate forward (v8/c68dae22972b): a, b [{M},{N}] bf16 -> bf16(silu(a)) * b bf16"),
-        "bwd": (4, 2, "kp_swiglu_bwd_bf16", "swiglu_bwd_vec",
+        "bwd": (4, 2, "kp_swiglu_bwd_bf16", "swiglu_vec",
                 "SwiGLU gate backward (v8/385e1beb9bb9): g, silu(a), b, a [{M},{N}] bf16 -> "
                 "db = g*silu(a), da = silu_backward(g*b, a) bf16"),
-        "silu": (1, 1, "kp_silu_bf16", "silu_vec", "SiLU (v7/58e7a4d6cde3): a [{M},{N}] bf16 -> silu(a) bf16"),
-        "fwdbwd": (3, 3, "kp_swiglu_fwd_bwd_bf16", "swiglu_fwd_bwd_vec",
+        "silu": (1, 1, "kp_silu_bf16", "swiglu_vec", "SiLU (v7/58e7a4d6cde3): a [{M},{N}] bf16 -> silu(a) bf16"),
+        "fwdbwd": (3, 3, "kp_swiglu_fwd_bwd_bf16", "swiglu_vec",
                    "SwiGLU gate forward recomputed with its backward (v6/182d2dcd0652): a, b, g [{M},{N}] bf16 -> "
                    "h = silu(a)*b, db = g*silu(a), da = silu_backward(g*b, a) bf16"),
     }

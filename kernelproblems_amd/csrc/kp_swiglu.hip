@@ -13,14 +13,16 @@
 // bf16 roundings where the eager op sequence materialises a bf16 tensor.
 //
 // Pure streaming: every element is read and written exactly once, so the
-// kernels are HBM-bound one-shot grids.  A block owns 4 x 256 consecutive
+// kernels are HBM-bound one-shot grids.  A block owns PER x 256 consecutive
 // 16-byte chunks (8 bf16 each) of every array; thread t holds chunks
 // t + 256 u, so each wave64 load or store moves 1 KiB of consecutive bytes.
 // All loads of a chunk group are issued before any math (one wait), loads and
-// stores are non-temporal.  Row-strided views run as rows of whole blocks
-// (block -> (row, column segment)); contiguous arrays run as one flat row.
-// Shapes whose rows, strides or pointers are not 16-byte granular take a
-// scalar grid-stride kernel with the same arithmetic.
+// stores are non-temporal.  Contiguous arrays run as one flat row; row-strided
+// views number the chunks of all rows consecutively, so that no block is cut
+// short by a row's end.  Rows and pointers may lie at any 2-byte address; the
+// elements past a row's last whole chunk are read with the 8 that end the row
+// and stored one by one.  Rows of fewer than 8 elements take a scalar grid-stride
+// kernel with the same arithmetic.
 #include "kp_common.hpp"
 #include "kp_internal.hpp"
 
@@ -28,9 +30,6 @@ namespace kp {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kPer = 4;                                    // chunks per thread per array
-constexpr int64_t kBlockChunks = (int64_t)kThreads * kPer;  // 16-byte chunks per block per array
-
 // ------------------------------------------------------------------ math
 // The eager formulas, evaluated in fp32 the way torch's silu / silu_backward
 // kernels do (expf, IEEE division, this operation order).
@@ -130,68 +129,86 @@ __device__ __forceinline__ void apply8(const u32x4* in, u32x4* out) {
 }
 
 // ------------------------------------------------------------------ 16-byte path
-// Arrays are [rows, cpr] in 16-byte chunks with per-array row strides (in
-// chunks).  Block b covers row b / bpr, chunks [(b % bpr) * kBlockChunks, +kBlockChunks).
+// Arrays of rows of n elements, cpr = ceil(n / 8) chunks each (flat: one row).
 struct VecArgs {
-  const u32x4* in[4];
-  u32x4* out[3];
-  int64_t in_rs[4], out_rs[3];  // row strides in chunks
-  int64_t cpr;                  // chunks per row
-  int bpr;                      // blocks per row
+  const uint16_t* in[4];
+  uint16_t* out[3];
+  int64_t in_rs[4], out_rs[3];  // row strides in elements (rows only)
+  int64_t n;
+  int64_t total;  // chunks of all rows (below 2^31 for rows)
+  Div32 cpr;      // rows only
 };
 
-template <bool FULL>
-__device__ __forceinline__ int64_t chunk_of(const VecArgs& a, int u, int64_t c0, bool& ok) {
-  const int64_t c = c0 + threadIdx.x + (int64_t)u * kThreads;
-  ok = FULL || c < a.cpr;
-  return ok ? c : 0;
+// Chunk k's row (0 when flat) and first column.
+template <bool ROWS>
+__device__ __forceinline__ void place(const VecArgs& a, int64_t k, uint32_t& row, int64_t& col) {
+  if constexpr (ROWS) {
+    row = div32((uint32_t)k, a.cpr);
+    col = (int64_t)(((uint32_t)k - row * a.cpr.d) * 8);
+  } else {
+    row = 0;
+    col = k * 8;
+  }
 }
 
-template <int OP, bool FULL>
-__device__ __forceinline__ void tile(const VecArgs& a, int64_t row, int64_t c0) {
+// One block's chunks.  WHOLE: flat and every chunk whole.  Otherwise the loads
+// of a chunk that its row's end cuts (or of one past the last) are moved back
+// into the row rather than predicated, so that the load batch issues
+// unbranched; only the stores are predicated, and a cut chunk's own elements
+// are stored one by one.
+template <int OP, int PER, bool ROWS, bool WHOLE>
+__device__ __forceinline__ void tile(const VecArgs& a, int64_t k0) {
   constexpr int NI = n_in(OP), NO = n_out(OP);
-  u32x4 v[NI][kPer];
-  int64_t c[kPer];
-  bool ok[kPer];
+  u32x4 v[NI][PER];
+  uint32_t row[PER];
+  int64_t col[PER];
 #pragma unroll
-  for (int u = 0; u < kPer; ++u) c[u] = chunk_of<FULL>(a, u, c0, ok[u]);
-#pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const u32x4* p = a.in[i] + row * a.in_rs[i];
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) v[i][u] = ld16_stream(p + c[u]);
+  for (int u = 0; u < PER; ++u) {
+    const int64_t k = k0 + threadIdx.x + u * kThreads;
+    place<ROWS>(a, WHOLE || k < a.total ? k : a.total - 1, row[u], col[u]);
   }
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int64_t c = WHOLE || col[u] + 8 <= a.n ? col[u] : a.n - 8;
+      v[i][u] = ld16u_stream(a.in[i] + (ROWS ? row[u] * a.in_rs[i] : 0) + c);
+    }
   // Every load of the tile is in flight before the first use: without this
   // fence the scheduler starts the math of chunk 0 after a few loads.
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int u = 0; u < kPer; ++u) {
+  for (int u = 0; u < PER; ++u) {
     u32x4 in[NI], r[NO];
 #pragma unroll
     for (int i = 0; i < NI; ++i) in[i] = v[i][u];
     apply8<OP>(in, r);
-    if (ok[u]) {
+    if (!WHOLE && k0 + threadIdx.x + u * kThreads >= a.total) continue;
+    if (WHOLE || col[u] + 8 <= a.n) {
 #pragma unroll
-      for (int o = 0; o < NO; ++o) st16_stream(a.out[o] + row * a.out_rs[o] + c[u], r[o]);
+      for (int o = 0; o < NO; ++o) st16u_stream(a.out[o] + (ROWS ? row[u] * a.out_rs[o] : 0) + col[u], r[o]);
+    } else {
+      const int skip = (int)(col[u] + 8 - a.n);  // 1..7 elements of the chunk before
+#pragma unroll
+      for (int o = 0; o < NO; ++o) {
+        uint16_t* q = a.out[o] + (ROWS ? row[u] * a.out_rs[o] : 0) + (a.n - 8);
+#pragma unroll
+        for (int e = 1; e < 8; ++e)
+          if (e >= skip) q[e] = (uint16_t)(r[o][e / 2] >> (e % 2 * 16));
+      }
     }
   }
 }
 
-// Loads of a partial tile are clamped to chunk 0 of the row (always in
-// bounds) rather than predicated, so the load batch issues unbranched; only
-// the stores are predicated.
-template <int OP>
-__device__ __forceinline__ void vec_body(const VecArgs& a) {
-  const int row = (int)blockIdx.x / a.bpr;
-  const int64_t c0 = (int64_t)((int)blockIdx.x - row * a.bpr) * kBlockChunks;
-  if (c0 + kBlockChunks <= a.cpr) tile<OP, true>(a, row, c0);
-  else tile<OP, false>(a, row, c0);
+template <int OP, int PER, bool ROWS>
+__global__ __launch_bounds__(kThreads) void swiglu_vec(VecArgs a) {
+  constexpr int64_t kBlock = (int64_t)kThreads * PER;
+  const int64_t k0 = (int64_t)blockIdx.x * kBlock;
+  if constexpr (!ROWS) {
+    if ((k0 + kBlock) * 8 <= a.n) return tile<OP, PER, ROWS, true>(a, k0);
+  }
+  tile<OP, PER, ROWS, false>(a, k0);
 }
-
-__global__ __launch_bounds__(kThreads) void swiglu_fwd_vec(VecArgs a) { vec_body<kFwd>(a); }
-__global__ __launch_bounds__(kThreads) void swiglu_bwd_vec(VecArgs a) { vec_body<kBwd>(a); }
-__global__ __launch_bounds__(kThreads) void silu_vec(VecArgs a) { vec_body<kSilu>(a); }
-__global__ __launch_bounds__(kThreads) void swiglu_fwd_bwd_vec(VecArgs a) { vec_body<kFwdBwd>(a); }
 
 // ------------------------------------------------------------------ scalar path
 struct ScalarArgs {
@@ -224,12 +241,13 @@ __global__ __launch_bounds__(kThreads) void swiglu_fwd_bwd_scalar(ScalarArgs a) 
 // ------------------------------------------------------------------ host side
 // Validates and launches one pointwise op over nin inputs / nout outputs of an
 // [M, N] bf16 matrix (unit inner stride, row strides in elements).
+template <bool ROWS>
 const void* vec_kernel(int op) {
   switch (op) {
-    case kFwd: return reinterpret_cast<const void*>(swiglu_fwd_vec);
-    case kBwd: return reinterpret_cast<const void*>(swiglu_bwd_vec);
-    case kSilu: return reinterpret_cast<const void*>(silu_vec);
-    default: return reinterpret_cast<const void*>(swiglu_fwd_bwd_vec);
+    case kFwd: return reinterpret_cast<const void*>(swiglu_vec<kFwd, 1, ROWS>);
+    case kBwd: return reinterpret_cast<const void*>(swiglu_vec<kBwd, 1, ROWS>);
+    case kSilu: return reinterpret_cast<const void*>(swiglu_vec<kSilu, 1, ROWS>);
+    default: return reinterpret_cast<const void*>(swiglu_vec<kFwdBwd, 1, ROWS>);
   }
 }
 
@@ -258,38 +276,40 @@ int launch_pointwise(const char* who, int op, const void* const* in, const int64
   }
   if (M > (((int64_t)1 << 62) / N)) return fail(KP_EUNSUPPORTED, "%s: [%lld, %lld] too large", who, (long long)M, (long long)N);
 
-  bool vec = (N % 8) == 0;
   bool flat = true;  // every array is one contiguous run of M*N elements
-  for (int i = 0; i < nin; ++i) {
-    vec = vec && aligned16(in[i]) && (M == 1 || in_rs[i] % 8 == 0);
-    flat = flat && (M == 1 || in_rs[i] == N);
-  }
-  for (int i = 0; i < nout; ++i) {
-    vec = vec && aligned16(out[i]) && (M == 1 || out_rs[i] % 8 == 0);
-    flat = flat && (M == 1 || out_rs[i] == N);
-  }
-  if (vec) {
+  for (int i = 0; i < nin; ++i) flat = flat && (M == 1 || in_rs[i] == N);
+  for (int i = 0; i < nout; ++i) flat = flat && (M == 1 || out_rs[i] == N);
+  const int64_t n = flat ? M * N : N, rows = flat ? 1 : M, cpr = ceil_div(n, 8);
+  if (n >= 8 && (flat || cpr <= 0x7fff0000LL / rows)) {
     VecArgs a{};
-    int64_t rows = M, cpr = N / 8;
-    if (flat) {
-      rows = 1;
-      cpr = M * N / 8;
-    }
     for (int i = 0; i < nin; ++i) {
-      a.in[i] = static_cast<const u32x4*>(in[i]);
-      a.in_rs[i] = flat ? 0 : in_rs[i] / 8;
+      a.in[i] = static_cast<const uint16_t*>(in[i]);
+      a.in_rs[i] = in_rs[i];
     }
     for (int i = 0; i < nout; ++i) {
-      a.out[i] = static_cast<u32x4*>(out[i]);
-      a.out_rs[i] = flat ? 0 : out_rs[i] / 8;
+      a.out[i] = static_cast<uint16_t*>(out[i]);
+      a.out_rs[i] = out_rs[i];
     }
-    a.cpr = cpr;
-    const int64_t bpr = ceil_div(cpr, kBlockChunks);
-    const int64_t blocks = bpr * rows;
+    a.n = n;
+    a.total = cpr * rows;
+    if (!flat) a.cpr = make_div32((uint32_t)cpr);
+    // One chunk per thread: many short blocks keep the last round of blocks
+    // short and mix the reads and writes of the chip better.  Measured on
+    // MI355X, one / four chunks per thread (us): forward [8192, 14336] 109.6 /
+    // 110.1, recompute [8192, 14336] 237 / 248, [2049, 5464] 24.7 / 29.6,
+    // halves of odd width [2049, 2 x 5461] 28.5 / 34.3 (scalar kernel 38.1),
+    // [16, 14336] 4.2 / 7.2.  Only the flat backward's four reads and two
+    // writes stream better four at a time once they are large: [2048, 14336]
+    // 58.0 / 59.7, [3072, 14336] 88.1 / 88.0, [4096, 14336] 119.5 / 116.4,
+    // [8192, 14336] 240 / 229.
+    const int per = flat && op == kBwd && a.total >= (int64_t)6 << 20 ? 4 : 1;
+    const int64_t blocks = ceil_div(a.total, (int64_t)kThreads * per);
     if (blocks > 0x7fffffffLL) return fail(KP_EUNSUPPORTED, "%s: too many blocks for one launch", who);
-    a.bpr = (int)bpr;
+    const void* fk = per == 4 ? reinterpret_cast<const void*>(swiglu_vec<kBwd, 4, false>)
+                     : flat   ? vec_kernel<false>(op)
+                              : vec_kernel<true>(op);
     void* args[] = {&a};
-    launch_dominant_raw(vec_kernel(op), dim3((unsigned)blocks), dim3(kThreads), args, 0, stream);
+    launch_dominant_raw(fk, dim3((unsigned)blocks), dim3(kThreads), args, 0, stream);
     return check_launch(who);
   }
   ScalarArgs a{};
