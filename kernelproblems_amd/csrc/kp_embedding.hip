@@ -5,7 +5,10 @@
 // Zipf-distributed ids hit the same rows repeatedly; output rows are written
 // with non-temporal stores.
 //
-// Backward pipeline (four launches on one stream, no float atomics).  The
+// Backward pipeline (two to four launches on one stream, no float atomics:
+// K1 does K2's work for a single chunk of tokens, and a single window needs
+// no K4).  Rows may lie at any address (D >= 4, D >= 8 forward; narrower rows
+// take scalar kernels).  The
 // token ids are sorted by (id, token) in 2048-token chunks and ranked
 // globally; the dense [V, D] result is then written by window blocks (summed
 // runs) and zero blocks (untouched rows).  The first three launches are
@@ -32,8 +35,8 @@
 //                        x 1024 columns: each run piece inside a window is
 //                        summed in ascending token order (fp32) and written as
 //                        the output row when the run lies inside the window,
-//                        else as an fp32 piece row.  Zero blocks: 1024 zero
-//                        columns of each untouched row of the rest.
+//                        else as an fp32 piece row.  Zero blocks: the untouched
+//                        rows of the rest.
 //   K4 emb_combine     : runs that span windows: the window holding the run's
 //                        start adds the pieces in window order and writes the
 //                        row.  Zero blocks: the untouched rows of the last share.
@@ -51,7 +54,7 @@ namespace kp {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kChunk = 2048;   // keys per K1 block (256 threads x 8)
+constexpr int kChunk = 2048;   // keys per K1 block (1024 threads x 2)
 constexpr int kChunkBits = 11;
 constexpr int kWin = 32;       // sorted positions per K3 window item
 constexpr uint32_t kSentinel = 0xffffffffu;
@@ -101,7 +104,7 @@ __global__ __launch_bounds__(kThreads) void emb_fwd_vec(EmbFwdArgs a) {
   for (; c0 + 512 * U <= a.D; c0 += 512 * U) {
     u32x4 v[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) v[u] = ld16(src + c0 + (u * 64 + lane) * 8);
+    for (int u = 0; u < U; ++u) v[u] = ld16u(src + c0 + (u * 64 + lane) * 8);
     // all eight loads, then all eight masks, then the eight stores: the
     // chunk's 8 KB leave as one burst (stores interleaved with the waits for
     // the loads took 33.2 against 31.2 us at C3)
@@ -110,24 +113,27 @@ __global__ __launch_bounds__(kThreads) void emb_fwd_vec(EmbFwdArgs a) {
     for (int u = 0; u < U; ++u) v[u] &= m;
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < U; ++u) st16_stream(dst + c0 + (u * 64 + lane) * 8, v[u]);
+    for (int u = 0; u < U; ++u) st16u_stream(dst + c0 + (u * 64 + lane) * 8, v[u]);
   }
-  if (c0 < a.D) {  // the last partial chunk of a row whose width is not a multiple of 4096
+  if (c0 < a.D) {
+    // The rest of a row whose width is not a multiple of 4096.  The chunk that
+    // crosses the row's end is the row's last 8 elements (D >= 8): those that
+    // the lane before also copies are stored twice, the same bits.
     u32x4 v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int64_t c = c0 + (int64_t)(u * 64 + lane) * 8;
-      v[u] = c < a.D ? ld16(src + c) : u32x4{0u, 0u, 0u, 0u};
+      v[u] = c < a.D ? ld16u(src + (c < a.D - 8 ? c : a.D - 8)) : u32x4{0u, 0u, 0u, 0u};
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int64_t c = c0 + (int64_t)(u * 64 + lane) * 8;
-      if (c < a.D) st16_stream(dst + c, v[u] & m);
+      if (c < a.D) st16u_stream(dst + (c < a.D - 8 ? c : a.D - 8), v[u] & m);
     }
   }
 }
 
-// Any row width or alignment: one bf16 per lane access.
+// Rows of fewer than 8 columns: one bf16 per lane access.
 __global__ __launch_bounds__(kThreads) void emb_fwd_scalar(EmbFwdArgs a) {
   const int lane = threadIdx.x & 63;
   const int64_t w0 = (int64_t)blockIdx.x * (kThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -176,10 +182,15 @@ struct EmbBwdArgs {
 };
 
 // Rows [lo, hi) of the zero fill carried by one launch; `cond` skips rows
-// whose bit is set in the touched-row bitmap.
+// whose bit is set in the touched-row bitmap.  Threads take units of `rep`
+// 16-byte chunks: numbered over the share's bytes when unconditional, per row
+// (upr units each) when not.  rep is 1 unless a share has 2^31 chunks.
 struct ZeroShare {
   int64_t lo, hi;
   int cond;
+  int rep;
+  int64_t units;  // below 2^31 when conditional
+  Div32 upr;
 };
 
 // Column ownership in the dense writer: a block handles one 1024-column chunk
@@ -188,20 +199,26 @@ struct ZeroShare {
 // covers one contiguous span of the row.
 constexpr int kColStep = kThreads * 4;
 
+// Rows lie at any 2-byte (grad, bf16 output) or 4-byte (fp32) address.
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2_u __attribute__((ext_vector_type(2), aligned(2)));
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 
 __device__ __forceinline__ u32x2 ld8_stream(const void* p) {
-  return __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(p));
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x2_u*>(p));
+}
+__device__ __forceinline__ void st16fu_stream(float* p, const f32x4& v) {
+  __builtin_nontemporal_store(v, reinterpret_cast<f32x4_u*>(p));
 }
 
 // Stores 4 consecutive output values (fp32 or bf16) at column c of row r.
 __device__ __forceinline__ void store_out4(const EmbBwdArgs& a, int64_t r, int64_t c, f32x4 v) {
   if (a.out_bf16) {
     const u32x2 pk = {pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
-    __builtin_nontemporal_store(pk, reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.out) + r * a.D + c));
+    __builtin_nontemporal_store(pk, reinterpret_cast<u32x2_u*>(static_cast<uint16_t*>(a.out) + r * a.D + c));
   } else {
     if (a.round_bf16) v = f32x4{round_bf(v[0]), round_bf(v[1]), round_bf(v[2]), round_bf(v[3])};
-    st16f_stream(static_cast<float*>(a.out) + r * a.D + c, v);
+    st16fu_stream(static_cast<float*>(a.out) + r * a.D + c, v);
   }
 }
 __device__ __forceinline__ void store_out1(const EmbBwdArgs& a, int64_t r, int64_t c, float v) {
@@ -212,200 +229,324 @@ __device__ __forceinline__ void store_out1(const EmbBwdArgs& a, int64_t r, int64
   }
 }
 
-// Zero block zb of a share: 1024 columns of one row (skipped when the share
-// is conditional and the row is touched).  The block's threads store one
-// 16-byte (or 8-byte bf16) vector each.
-template <bool VEC>
-__device__ __forceinline__ void zero_block(const EmbBwdArgs& a, const ZeroShare& z, int64_t zb) {
-  const int64_t nq = (a.D + kColStep - 1) / kColStep;
-  const int64_t r = z.lo + zb / nq, q = zb % nq;
-  if (r >= z.hi || r >= a.V) return;
-  if (z.cond && ((a.bitmap[r >> 5] >> (r & 31)) & 1u)) return;
-  if constexpr (VEC) {
-    const int64_t c = q * kColStep + (int64_t)threadIdx.x * 4;
-    if (c < a.D) store_out4(a, r, c, f32x4{0.f, 0.f, 0.f, 0.f});
+__device__ __forceinline__ bool touched(const EmbBwdArgs& a, int64_t r) {
+  return ((a.bitmap[r >> 5] >> (r & 31)) & 1u) != 0;
+}
+
+// n zeros (a 16-byte chunk) from element e of the output; fewer than a chunk
+// one by one.
+__device__ __forceinline__ void zero_chunk(const EmbBwdArgs& a, int64_t e, int n) {
+  if (a.out_bf16) {
+    uint16_t* q = static_cast<uint16_t*>(a.out) + e;
+    if (n == 8) st16u_stream(q, u32x4{0u, 0u, 0u, 0u});
+    else
+      for (int i = 0; i < n; ++i) q[i] = 0;
   } else {
-    for (int64_t c = q * kColStep + threadIdx.x; c < min(a.D, (q + 1) * kColStep); c += kThreads) store_out1(a, r, c, 0.f);
+    float* q = static_cast<float*>(a.out) + e;
+    if (n == 4) st16fu_stream(q, f32x4{0.f, 0.f, 0.f, 0.f});
+    else
+      for (int i = 0; i < n; ++i) q[i] = 0.f;
   }
+}
+// Chunk k of the elements [base, base + len): the last one is moved back to
+// end with them (zeros twice) unless they are fewer than a chunk.
+__device__ __forceinline__ void zero_part(const EmbBwdArgs& a, int64_t base, int64_t len, int64_t k) {
+  const int per = a.out_bf16 ? 8 : 4;
+  if (k * per >= len) return;
+  if (len < per) zero_chunk(a, base, (int)len);
+  else zero_chunk(a, base + (k * per < len - per ? k * per : len - per), per);
+}
+
+// Zero block zb of a share: NT units, i.e. one 16-byte store per thread
+// whatever the row width or output type (a pure write stream is fastest in 4
+// KiB blocks of single stores, and a block's few scalar instructions count:
+// a block that found its row by a 64-bit multiply-high and tested the bitmap
+// per lane took the fp32 [128256, 4096] fill from 6.6 to 4.4 TB/s).  Against blocks of
+// 1024 columns of one row (8-byte stores for bf16, a half-empty last block),
+// the bf16 gradient [32003, 2560] of 1501 tokens takes 39 us in three launches
+// in place of 63 us in four.
+template <int NT = kThreads>
+__device__ __forceinline__ void zero_block(const EmbBwdArgs& a, const ZeroShare& z, int64_t zb) {
+  const int64_t u0 = zb * NT;
+  if (!z.cond) {
+    const int64_t u = u0 + threadIdx.x;
+    for (int i = 0; i < z.rep; ++i) zero_part(a, z.lo * a.D, (z.hi - z.lo) * a.D, u * z.rep + i);
+    return;
+  }
+  uint32_t r = div32((uint32_t)u0, z.upr);
+  if ((uint32_t)u0 + NT <= (r + 1) * z.upr.d) {  // the whole block in one row: one scalar test
+    if (z.lo + r >= z.hi || touched(a, z.lo + r)) return;
+  } else {
+    const uint32_t u = (uint32_t)u0 + threadIdx.x;
+    r = div32(u, z.upr);
+    if (u >= z.units || touched(a, z.lo + r)) return;
+  }
+  const int64_t k = ((uint32_t)u0 + threadIdx.x - r * z.upr.d) * (int64_t)z.rep;
+  for (int i = 0; i < z.rep; ++i) zero_part(a, (z.lo + r) * a.D, a.D, k + i);
 }
 
 // ---- K1: sort each chunk of keys (bitonic, ascending) --------------------
-// Thread t holds positions 8t..8t+7.  Stages with partner distance j < 8 are
-// register min/max, 8 <= j < 512 exchange within the wave (lane t ^ j/8),
-// j >= 512 go through LDS with block barriers.  Blocks past nchunks are the
-// launch's zero share.
-template <bool VEC>
-__global__ __launch_bounds__(kThreads) void emb_sort_chunks(EmbBwdArgs a, ZeroShare z) {
+// 1024 threads, thread t holding positions 2t and 2t + 1: the sort is one
+// block's chain of 66 dependent stages, bound by its CU's VALU (16 waves; the
+// launch with few zero blocks takes 10 us, 14 us with 8 positions in each of
+// 256 threads).  Partner distance 1 is in the thread, 2..64 exchange within the wave
+// (lane t ^ j/2), 128 and more go through LDS, two buffers in turn (one
+// barrier a stage).  Blocks past nchunks are the launch's zero share.
+//
+// RANK (one chunk of tokens, a vocabulary of up to kRankMaxV rows): the sorted
+// chunk is the global order, so this launch also finds the run bounds, by
+// binary search in LDS, and builds the touched-row bitmap there -- K2's work
+// without its launch and its chain of cached loads (1501 tokens: 11 us for
+// both against 15 + 14).  Only as many positions as there are tokens are
+// sorted (rounded up to a power of two): 3.5 us for 16 tokens.
+constexpr int kSortThreads = 1024;
+constexpr int64_t kRankMaxV = 131072;  // 16 KiB of bitmap
+
+// Lane l's value of lane l ^ M.
+template <int M>
+__device__ __forceinline__ uint32_t xor_lane(uint32_t v) {
+  if constexpr (M == 1) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true);   // quad_perm [1,0,3,2]
+  if constexpr (M == 2) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true);   // quad_perm [2,3,0,1]
+  if constexpr (M == 8) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xF, 0xF, true);  // row_ror:8
+  return (uint32_t)__shfl_xor((int)v, M, 64);
+}
+
+// Position i's key after comparing with `o`, position i ^ j's, in stage k.
+__device__ __forceinline__ uint32_t keep(uint32_t v, uint32_t o, int i, int j, int k) {
+  return ((i & j) == 0) == ((i & k) == 0) ? min(v, o) : max(v, o);
+}
+
+template <bool RANK>
+__global__ __launch_bounds__(kSortThreads) void emb_sort_chunks(EmbBwdArgs a, ZeroShare z) {
   if ((int64_t)blockIdx.x >= a.nchunks) {
-    zero_block<VEC>(a, z, (int64_t)blockIdx.x - a.nchunks);
+    zero_block<kSortThreads>(a, z, (int64_t)blockIdx.x - a.nchunks);
     return;
   }
-  __shared__ uint32_t s[kChunk];
+  __shared__ uint32_t s[2][kChunk];
   const int tid = threadIdx.x;
   const int64_t base = (int64_t)blockIdx.x * kChunk;
 
-  // clear this block's share of the bitmap (K2 sets bits after this kernel)
   const int64_t nwords = (a.V + 31) / 32;
-  const int64_t per = (nwords + a.nchunks - 1) / a.nchunks;
-  for (int64_t w = blockIdx.x * per + tid; w < min(nwords, (int64_t)(blockIdx.x + 1) * per); w += kThreads)
-    a.bitmap[w] = 0u;
+  extern __shared__ uint32_t bits[];  // RANK: the bitmap
+  if constexpr (RANK) {
+    for (int w = tid; w < (int)nwords; w += kSortThreads) bits[w] = 0u;
+  } else {
+    // clear this block's share of the bitmap (K2 sets bits after this kernel)
+    const int64_t per = (nwords + a.nchunks - 1) / a.nchunks;
+    for (int64_t w = blockIdx.x * per + tid; w < min(nwords, (int64_t)(blockIdx.x + 1) * per); w += kSortThreads)
+      a.bitmap[w] = 0u;
+  }
 
-  // Element e of thread tid is token base + e * 256 + tid (coalesced index
-  // loads); the keys are unique within the chunk, so their placement does
-  // not change the sorted result.  All 8 index loads go out before any of
-  // them is used: the error-flag store below may alias the index buffer as
-  // far as the compiler knows, so loading and checking one index at a time
-  // serializes 8 memory round trips.  Slots past the end re-read the last
-  // index (never used); with no tokens at all (the index buffer may be NULL)
-  // nothing is read.  The index width is tested once for the whole batch (a
-  // per-load branch makes the compiler wait after every int32 load).
-  int64_t id8[8];
+  // Element e of thread tid is token base + e * 1024 + tid (coalesced index
+  // loads; RANK: token tid * 2 + e, its place in the sort); the keys are
+  // unique within the chunk, so their placement does not change the sorted
+  // result.  Both index loads go out before either is used: the error-flag
+  // store below may alias the index buffer as far as the compiler knows.
+  // Slots past the end re-read the last index (never used); with no tokens at
+  // all (the index buffer may be NULL) nothing is read.
+  auto place = [&](int e) { return RANK ? tid * 2 + e : e * kSortThreads + tid; };
+  int64_t id2[2] = {0, 0};
   if (a.T > 0 && a.ib == 8) {
     const int64_t* ix = static_cast<const int64_t*>(a.idx);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int64_t t = base + e * kThreads + tid;
-      id8[e] = ix[t < a.T ? t : a.T - 1];
+    for (int e = 0; e < 2; ++e) {
+      const int64_t t = base + place(e);
+      id2[e] = ix[t < a.T ? t : a.T - 1];
     }
   } else if (a.T > 0) {
     const int32_t* ix = static_cast<const int32_t*>(a.idx);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int64_t t = base + e * kThreads + tid;
-      id8[e] = ix[t < a.T ? t : a.T - 1];
+    for (int e = 0; e < 2; ++e) {
+      const int64_t t = base + place(e);
+      id2[e] = ix[t < a.T ? t : a.T - 1];
     }
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) id8[e] = 0;
   }
-  uint32_t k8[8];
+  uint32_t k2[2];
   int nvalid = 0;
   bool bad = false;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const int64_t t = base + e * kThreads + tid;
-    const int64_t id = id8[e];
+  for (int e = 0; e < 2; ++e) {
+    const int64_t id = id2[e];
     uint32_t key = kSentinel;
-    if (t < a.T) {
+    if (base + place(e) < a.T) {
       const bool in_range = id >= 0 && id < a.v_all;
       bad |= !in_range;
       const int64_t rel = id - a.id_lo;  // ids of other slabs contribute nothing to this pass
       if (in_range && rel >= 0 && rel < a.V && id != a.padding_idx) {
-        key = ((uint32_t)rel << kChunkBits) | (uint32_t)(e * kThreads + tid);
+        key = ((uint32_t)rel << kChunkBits) | (uint32_t)place(e);
         ++nvalid;
       }
     }
-    k8[e] = key;
+    k2[e] = key;
   }
   if (bad && a.err) *a.err = 1;
 
+  const int i0 = 2 * tid;
+  int buf = 0;
+#define KP_WAVE_STAGE(J)                                          \
+  if (j == (J)) {                                                 \
+    k2[0] = keep(k2[0], xor_lane<(J) / 2>(k2[0]), i0, (J), k);    \
+    k2[1] = keep(k2[1], xor_lane<(J) / 2>(k2[1]), i0, (J), k);    \
+  }
 #pragma unroll
   for (int k = 2; k <= kChunk; k <<= 1) {
+    // positions from T on hold sentinels: the runs of k >= 2 T positions are in order already
+    if (RANK && k >= 2 * a.T) break;
 #pragma unroll
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      if (j >= 512) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s[tid * 8 + e] = k8[e];
+    for (int j = k >> 1; j > 1; j >>= 1) {
+      if (j >= 128) {
+        s[buf][i0] = k2[0];
+        s[buf][i0 + 1] = k2[1];
         __syncthreads();
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int i = tid * 8 + e, l = i ^ j;
-          const uint32_t o = s[l];
-          const bool take_min = ((i < l) == ((i & k) == 0));
-          k8[e] = take_min ? min(k8[e], o) : max(k8[e], o);
-        }
-        __syncthreads();
-      } else if (j >= 8) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int i = tid * 8 + e, l = i ^ j;
-          const uint32_t o = (uint32_t)__shfl_xor((int)k8[e], j >> 3, 64);
-          const bool take_min = ((i < l) == ((i & k) == 0));
-          k8[e] = take_min ? min(k8[e], o) : max(k8[e], o);
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          if (e & j) continue;
-          const int i = tid * 8 + e;
-          const bool up = (i & k) == 0;
-          const uint32_t x = k8[e], y = k8[e | j];
-          k8[e] = up ? min(x, y) : max(x, y);
-          k8[e | j] = up ? max(x, y) : min(x, y);
-        }
+        const int l = i0 ^ j;
+        k2[0] = keep(k2[0], s[buf][l], i0, j, k);
+        k2[1] = keep(k2[1], s[buf][l + 1], i0, j, k);
+        buf ^= 1;
       }
+      KP_WAVE_STAGE(64)
+      KP_WAVE_STAGE(32)
+      KP_WAVE_STAGE(16)
+      KP_WAVE_STAGE(8)
+      KP_WAVE_STAGE(4)
+      KP_WAVE_STAGE(2)
     }
+    const bool up = (i0 & k) == 0;
+    const uint32_t x = k2[0], y = k2[1];
+    k2[0] = up ? min(x, y) : max(x, y);
+    k2[1] = up ? max(x, y) : min(x, y);
   }
-  uint32_t* dst = a.keys_chunk + base + tid * 8;
-  *reinterpret_cast<u32x4*>(dst) = u32x4{k8[0], k8[1], k8[2], k8[3]};
-  *reinterpret_cast<u32x4*>(dst + 4) = u32x4{k8[4], k8[5], k8[6], k8[7]};
+#undef KP_WAVE_STAGE
   // valid keys of the chunk (integer sum: order-independent)
   __shared__ int s_cnt;
+  uint32_t* v = s[buf];  // not the buffer that a slower wave may still read
   if (tid == 0) s_cnt = 0;
+  if constexpr (RANK) {
+    v[i0] = k2[0];
+    v[i0 + 1] = k2[1];
+  } else {
+    *reinterpret_cast<uint64_t*>(a.keys_chunk + base + i0) = (uint64_t)k2[1] << 32 | k2[0];
+  }
   __syncthreads();
   if (nvalid) atomicAdd(&s_cnt, nvalid);
+  if constexpr (RANK) {
+    // Per position: #keys of smaller ids and #keys of ids up to its own (the
+    // searches of both positions advance in lockstep).
+    int pl[2] = {0, 0}, ph[2] = {0, 0};
+#pragma unroll
+    for (int step = kChunk >> 1; step > 0; step >>= 1) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const uint32_t q_lo = k2[e] & ~(uint32_t)(kChunk - 1);
+        if (v[pl[e] + step - 1] < q_lo) pl[e] += step;
+        if (v[ph[e] + step - 1] < q_lo + kChunk) ph[e] += step;  // a valid id is below 2^21 - 1: no overflow
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      if (k2[e] == kSentinel) continue;
+      const uint32_t id = k2[e] >> kChunkBits;
+      const int p = i0 + e;
+      const int lo = pl[e] + (v[pl[e]] < (id << kChunkBits) ? 1 : 0);
+      const int hi = ph[e] + (v[ph[e]] < ((id + 1) << kChunkBits) ? 1 : 0);
+      a.sid[p] = id;
+      a.stok[p] = k2[e] & (uint32_t)(kChunk - 1);
+      a.run_lo[p] = lo;
+      a.run_hi[p] = hi;
+      if (p == lo) atomicOr(bits + (id >> 5), 1u << (id & 31));
+    }
+  }
   __syncthreads();
-  if (tid == 0) a.chunk_valid[blockIdx.x] = s_cnt;
+  if constexpr (RANK) {
+    for (int w = tid; w < (int)nwords; w += kSortThreads) a.bitmap[w] = bits[w];
+    if (tid == 0) a.hdr->n_valid = s_cnt;
+  } else {
+    if (tid == 0) a.chunk_valid[blockIdx.x] = s_cnt;
+  }
 }
 
 // ---- K2: global rank and run bounds of every valid key -------------------
 // Position i of the chunk-sorted keys (chunk c, place p in it) holds id v.
 // Per chunk o: lo_o = #keys of ids < v, hi_o = #keys of ids <= v (two
-// branch-free binary searches; the 11-step searches of a batch of chunks
-// advance in lockstep so their loads overlap).  Run bounds: lo = sum lo_o,
-// hi = sum hi_o.  Rank in (id, token) order: p + sum_{o < c} hi_o +
-// sum_{o > c} lo_o -- equal ids of earlier chunks are earlier tokens.  The
-// sorted chunks (a few hundred KB at most) are read through the caches.
-constexpr int kRankBatch = 8;
+// branch-free binary searches).  Run bounds: lo = sum lo_o, hi = sum hi_o.
+// Rank in (id, token) order: p + sum_{o < c} hi_o + sum_{o > c} lo_o -- equal
+// ids of earlier chunks are earlier tokens.
+// The launch is a chain of dependent loads, so a block first copies every
+// 32nd key of (up to 64) chunks to LDS: a search takes 6 steps there and 5
+// in the cached keys instead of 11 cached loads one after another.  The
+// searches of a batch of chunks advance in lockstep so their loads overlap.
+constexpr int kRankBatch = 4;
+constexpr int kRankGroup = 32;                    // keys per sample
+constexpr int kRankSamples = kChunk / kRankGroup;  // 64 per chunk
+constexpr int kRankChunks = 64;                   // chunks sampled at a time
 
-template <bool VEC>
 __global__ __launch_bounds__(kThreads) void emb_rank(EmbBwdArgs a, int rank_blocks, ZeroShare z) {
   if ((int)blockIdx.x >= rank_blocks) {
-    zero_block<VEC>(a, z, (int64_t)blockIdx.x - rank_blocks);
+    zero_block(a, z, (int64_t)blockIdx.x - rank_blocks);
     return;
   }
+  __shared__ uint32_t samp[kRankChunks * kRankSamples];
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     int n = 0;
     for (int c = 0; c < a.nchunks; ++c) n += a.chunk_valid[c];
     a.hdr->n_valid = n;
   }
-  const int64_t total = (int64_t)a.nchunks * kChunk;
-  const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  if (i >= total) return;
+  const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;  // rank_blocks cover the keys exactly
   const uint32_t key = a.keys_chunk[i];
-  if (key == kSentinel) return;
   const int c = (int)(i / kChunk);
   const int p = (int)(i - (int64_t)c * kChunk);
   const uint32_t id = key >> kChunkBits;
   const uint32_t q_lo = id << kChunkBits, q_hi = (id + 1) << kChunkBits;  // id < 2^21 - 1: no overflow
   int64_t lo = 0, hi = 0, rank = p;
-  for (int o0 = 0; o0 < a.nchunks; o0 += kRankBatch) {
-    int pl[kRankBatch], ph[kRankBatch];
-#pragma unroll
-    for (int b = 0; b < kRankBatch; ++b) pl[b] = ph[b] = 0;
-#pragma unroll
-    for (int step = kChunk >> 1; step > 0; step >>= 1) {
+  for (int s0 = 0; s0 < a.nchunks; s0 += kRankChunks) {
+    const int ns = min(kRankChunks, a.nchunks - s0);
+    if (s0 > 0) __syncthreads();
+    for (int x = threadIdx.x; x < ns * kRankSamples; x += kThreads)
+      samp[x] = a.keys_chunk[((int64_t)s0 * kRankSamples + x) * kRankGroup + kRankGroup - 1];
+    __syncthreads();
+    if (key == kSentinel) continue;
+    for (int o0 = 0; o0 < ns; o0 += kRankBatch) {
+      int pl[kRankBatch], ph[kRankBatch];
 #pragma unroll
       for (int b = 0; b < kRankBatch; ++b) {
-        const int o = o0 + b < a.nchunks ? o0 + b : a.nchunks - 1;  // clamped: results of o >= nchunks unused
-        const uint32_t* v = a.keys_chunk + (int64_t)o * kChunk;
-        if (v[pl[b] + step - 1] < q_lo) pl[b] += step;
-        if (v[ph[b] + step - 1] < q_hi) ph[b] += step;
+        // groups of 32 keys wholly below the bound (the sample is a group's last key)
+        const uint32_t* v = samp + min(o0 + b, ns - 1) * kRankSamples;
+        int gl = 0, gh = 0;
+#pragma unroll
+        for (int step = kRankSamples >> 1; step > 0; step >>= 1) {
+          if (v[gl + step - 1] < q_lo) gl += step;
+          if (v[gh + step - 1] < q_hi) gh += step;
+        }
+        pl[b] = gl + (v[gl] < q_lo ? 1 : 0);
+        ph[b] = gh + (v[gh] < q_hi ? 1 : 0);
+      }
+      int el[kRankBatch], eh[kRankBatch];
+#pragma unroll
+      for (int b = 0; b < kRankBatch; ++b) el[b] = eh[b] = 0;
+#pragma unroll
+      for (int step = kRankGroup >> 1; step > 0; step >>= 1) {
+#pragma unroll
+        for (int b = 0; b < kRankBatch; ++b) {
+          // clamped: the results of o >= ns and of a chunk wholly below the bound are not used
+          const uint32_t* v = a.keys_chunk + (int64_t)(s0 + min(o0 + b, ns - 1)) * kChunk;
+          if (v[min(pl[b], kRankSamples - 1) * kRankGroup + el[b] + step - 1] < q_lo) el[b] += step;
+          if (v[min(ph[b], kRankSamples - 1) * kRankGroup + eh[b] + step - 1] < q_hi) eh[b] += step;
+        }
+      }
+#pragma unroll
+      for (int b = 0; b < kRankBatch; ++b) {
+        const int o = s0 + o0 + b;
+        if (o0 + b >= ns) break;
+        // the group's last key is not below the bound, so at most 31 of its keys are
+        const int cl = pl[b] * kRankGroup + (pl[b] < kRankSamples ? el[b] : 0);
+        const int ch = ph[b] * kRankGroup + (ph[b] < kRankSamples ? eh[b] : 0);
+        lo += cl;
+        hi += ch;
+        if (o < c) rank += ch;
+        else if (o > c) rank += cl;
       }
     }
-#pragma unroll
-    for (int b = 0; b < kRankBatch; ++b) {
-      const int o = o0 + b;
-      if (o >= a.nchunks) break;
-      const uint32_t* v = a.keys_chunk + (int64_t)o * kChunk;
-      const int cl = pl[b] + (v[pl[b]] < q_lo ? 1 : 0);
-      const int ch = ph[b] + (v[ph[b]] < q_hi ? 1 : 0);
-      lo += cl;
-      hi += ch;
-      if (o < c) rank += ch;
-      else if (o > c) rank += cl;
-    }
   }
+  if (key == kSentinel) return;
   if (rank >= a.T) return;  // impossible (ranks are a permutation); bounds the stores regardless
   a.sid[rank] = id;
   a.stok[rank] = (uint32_t)((int64_t)c * kChunk + (key & (kChunk - 1)));
@@ -431,7 +572,7 @@ __device__ __forceinline__ void emit_piece_row(const EmbBwdArgs& a, int64_t w, i
     if (row < a.V) store_out4(a, row, c, acc);
   } else {
     const int slot = lo < w0 ? 0 : 1;  // 0: continues from an earlier window; 1: run starts here
-    *reinterpret_cast<f32x4*>(a.pieces + (2 * w + slot) * a.D + c) = acc;
+    *reinterpret_cast<f32x4_u*>(a.pieces + (2 * w + slot) * a.D + c) = acc;
   }
 }
 __device__ __forceinline__ void emit_piece1(const EmbBwdArgs& a, int64_t w, int64_t w0, int64_t w1, int lo, int hi,
@@ -451,24 +592,32 @@ __device__ __forceinline__ void emit_piece1(const EmbBwdArgs& a, int64_t w, int6
 // loads per thread), and each column's additions run in ascending position
 // order.  Run boundaries are block-uniform (run_lo / run_hi of the position).
 template <bool VEC>
-__device__ void emb_do_window(const EmbBwdArgs& a, int64_t w, int64_t q, int n_valid) {
+__device__ void emb_do_window(const EmbBwdArgs& a, int64_t w, int64_t q) {
   const int64_t w0 = w * kWin;
-  const int64_t w1 = min((int64_t)n_valid, w0 + kWin);
   if constexpr (VEC) {
     constexpr int U = 16;
-    const int64_t col = q * kColStep + threadIdx.x * 4;
-    const bool on = col < a.D;
+    // The 4 columns that cross the row's end are its last 4 (D >= 4): those
+    // that another thread also owns are summed and stored twice, the same bits.
+    const int64_t cn = q * kColStep + threadIdx.x * 4;
+    const bool on = cn < a.D;
+    const int64_t col = cn < a.D - 4 ? cn : a.D - 4;
     // Lane i < np holds position w0 + i's token, run bounds and id, fetched
     // in one batch and read as scalars (readlane) by the loop: a window of
     // many short runs would otherwise wait for one dependent load of its
-    // bounds (and one of its id) per run.
-    const int np = (int)(w1 - w0);  // 1..kWin
+    // bounds (and one of its id) per run.  They are requested together with
+    // the number of valid positions, which only says how many of them count
+    // (the block is a chain of dependent loads; w0 < T).
     const int lane = threadIdx.x & 63;
-    const int64_t pl = w0 + (lane < np ? lane : np - 1);
-    const int tok_l = (int)token_of(a, pl);
-    const int lo_l = clamp_pos(a.run_lo[pl], n_valid);
-    const int hi_l = clamp_pos(a.run_hi[pl], n_valid);
+    const int64_t pl = min(w0 + (lane & (kWin - 1)), a.T - 1);
+    const uint32_t tok_r = a.stok[pl];
+    const int lo_r = a.run_lo[pl], hi_r = a.run_hi[pl];
     const int id_l = (int)a.sid[pl];
+    const int n_valid = (int)min((int64_t)max(a.hdr->n_valid, 0), a.T);
+    const int64_t w1 = min((int64_t)n_valid, w0 + kWin);
+    const int np = (int)(w1 - w0);  // up to kWin
+    if (np <= 0) return;
+    const int tok_l = (int64_t)tok_r < a.T ? (int)tok_r : 0;
+    const int lo_l = clamp_pos(lo_r, n_valid), hi_l = clamp_pos(hi_r, n_valid);
     int lo = (int)w0, hi = (int)w0;  // hi == w0: a run starts at the first position
     float cnt = 1.f;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -503,6 +652,8 @@ __device__ void emb_do_window(const EmbBwdArgs& a, int64_t w, int64_t q, int n_v
       }
     }
   } else {
+    const int n_valid = (int)min((int64_t)max(a.hdr->n_valid, 0), a.T);
+    const int64_t w1 = min((int64_t)n_valid, w0 + kWin);
     for (int64_t c = q * kColStep + threadIdx.x; c < min(a.D, (q + 1) * kColStep); c += kThreads) {
       int64_t r = w0;
       while (r < w1) {
@@ -529,13 +680,10 @@ __global__ __launch_bounds__(kThreads) void emb_dense(EmbBwdArgs a, int64_t n_wi
   const int64_t nq = (a.D + kColStep - 1) / kColStep;
   const int64_t b = blockIdx.x;
   if (b < n_win_blocks) {
-    const int n_valid = (int)min((int64_t)max(a.hdr->n_valid, 0), a.T);
-    const int64_t w = b / nq, q = b % nq;
-    if (w * kWin >= n_valid) return;
-    emb_do_window<VEC>(a, w, q, n_valid);
+    emb_do_window<VEC>(a, b / nq, b % nq);
     return;
   }
-  zero_block<VEC>(a, z, b - n_win_blocks);
+  zero_block(a, z, b - n_win_blocks);
 }
 
 // ---- K4: runs spanning windows, pieces added in window order ---------------
@@ -544,7 +692,7 @@ __global__ __launch_bounds__(kThreads) void emb_dense(EmbBwdArgs a, int64_t n_wi
 template <bool VEC>
 __global__ __launch_bounds__(kThreads) void emb_combine(EmbBwdArgs a, int comb_blocks, ZeroShare z) {
   if ((int)blockIdx.x >= comb_blocks) {
-    zero_block<VEC>(a, z, (int64_t)blockIdx.x - comb_blocks);
+    zero_block(a, z, (int64_t)blockIdx.x - comb_blocks);
     return;
   }
   const int n_valid = (int)min((int64_t)max(a.hdr->n_valid, 0), a.T);
@@ -560,15 +708,16 @@ __global__ __launch_bounds__(kThreads) void emb_combine(EmbBwdArgs a, int comb_b
     const int64_t row = row_of(a, lo);
     if (row >= a.V) continue;
     if constexpr (VEC) {
-      const int64_t c = q * kColStep + (int64_t)threadIdx.x * 4;
-      if (c >= a.D) continue;
-      f32x4 acc = *reinterpret_cast<const f32x4*>(a.pieces + (2 * w + 1) * a.D + c);
+      const int64_t cn = q * kColStep + (int64_t)threadIdx.x * 4;
+      if (cn >= a.D) continue;
+      const int64_t c = cn < a.D - 4 ? cn : a.D - 4;
+      f32x4 acc = *reinterpret_cast<const f32x4_u*>(a.pieces + (2 * w + 1) * a.D + c);
       constexpr int U = 16;
       for (int64_t w2 = w + 1; w2 <= wl; w2 += U) {
         f32x4 v[U];
 #pragma unroll
         for (int u = 0; u < U; ++u)
-          v[u] = (w2 + u <= wl) ? *reinterpret_cast<const f32x4*>(a.pieces + (2 * (w2 + u)) * a.D + c)
+          v[u] = (w2 + u <= wl) ? (f32x4) * reinterpret_cast<const f32x4_u*>(a.pieces + (2 * (w2 + u)) * a.D + c)
                                 : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -883,9 +1032,9 @@ Layout make_layout(int64_t T, int64_t V, int64_t D) {
 
 // Zero-fill share of each latency-chain launch, in MiB of output rows (K1,
 // K2: unconditional; K4: conditional), at least as long to stream as the
-// launch's own chain (~13-17 us each at the C3 configuration).  Measured on
-// MI355X at C3 (whole call): 96/96/64 MiB 357.1 us, 128/128/96 356.1 us,
-// 160/160/128 357.6 us, 256/256/192 360.9 us -- once the chains are hidden
+// launch's own chain (~10-13 us each at the C3 configuration).  Measured on
+// MI355X at C3 (whole call): 64/64/64 MiB 329.6 us, 96/96/64 327.9 us,
+// 128/128/96 329.2 us, 256/256/192 336.4 us, none 348.8 us -- once the chains are hidden
 // the pipeline is bound by HBM alone.  Tuning knobs: KP_EMB_ZERO_MB_SORT /
 // _RANK / _COMBINE.
 int64_t share_rows(const char* env, int64_t dflt_mb, int64_t row_bytes, int64_t cap_rows) {
@@ -914,6 +1063,55 @@ ChainLayout make_chain_layout(int64_t T, int64_t V, int64_t D) {
   return L;
 }
 
+// The zero fill of one slab split over the launches, from the top of the
+// vocabulary down (high ids are the rarely touched ones under the usual
+// frequency-ordered vocabularies): K1 [V - z1, V), K2 [V - z1 - z2, V - z1),
+// K4 [r3, V - z1 - z2), K3 [0, r3).  Without K2 (ranked in K1) K1 takes three
+// eighths, and without K4 (`combine` false) K3 takes its share.
+struct ZeroShares {
+  ZeroShare s1, s2, s3, s4;
+};
+ZeroShare make_share(int64_t lo, int64_t hi, int cond, int64_t row_bytes) {
+  ZeroShare z{lo, hi, cond, 1, 0, make_div32(1)};
+  for (;; z.rep *= 2) {
+    const int64_t upr = ceil_div(row_bytes, (int64_t)16 * z.rep);
+    z.units = cond ? upr * (hi - lo) : ceil_div((hi - lo) * row_bytes, (int64_t)16 * z.rep);
+    if (z.units > 0x7fff0000LL) continue;
+    if (cond) z.upr = make_div32((uint32_t)upr);
+    return z;
+  }
+}
+ZeroShares make_shares(int64_t V, int64_t row_bytes, bool ranked, bool combine) {
+  ZeroShares Z{};
+  const int64_t z1 = share_rows("KP_EMB_ZERO_MB_SORT", 96, row_bytes, ranked ? V * 3 / 8 : V / 4);
+  const int64_t z2 = ranked ? 0 : share_rows("KP_EMB_ZERO_MB_RANK", 96, row_bytes, V / 4);
+  const int64_t z4 = combine ? share_rows("KP_EMB_ZERO_MB_COMBINE", 64, row_bytes, V / 4) : 0;
+  Z.s1 = make_share(V - z1, V, 0, row_bytes);
+  Z.s2 = make_share(V - z1 - z2, V - z1, 0, row_bytes);
+  Z.s4 = make_share(V - z1 - z2 - z4, V - z1 - z2, 1, row_bytes);
+  Z.s3 = make_share(0, V - z1 - z2 - z4, 1, row_bytes);
+  return Z;
+}
+int64_t zero_blocks(const ZeroShare& z) { return ceil_div(z.units, kThreads); }
+
+// K1 (ranking too where it can) and K2.
+bool ranked_in_sort(const EmbBwdArgs& a) { return a.nchunks == 1 && a.V <= kRankMaxV; }
+int launch_sort(const char* who, const EmbBwdArgs& a, const ZeroShares& Z, bool first, hipStream_t s) {
+  const int64_t rank_blocks = ceil_div((int64_t)a.nchunks * kChunk, kThreads);
+  const int64_t g1 = a.nchunks + ceil_div(Z.s1.units, kSortThreads), g2 = rank_blocks + zero_blocks(Z.s2);
+  if (g1 > 0x7fffffffLL || g2 > 0x7fffffffLL) return fail(KP_EUNSUPPORTED, "%s: V * D too large for one launch", who);
+  if (ranked_in_sort(a)) {
+    KP_LAUNCH_SPAN(first, false, emb_sort_chunks<true>, dim3((unsigned)g1), dim3(kSortThreads),
+                   (size_t)ceil_div(a.V, 32) * 4, s, a, Z.s1);
+    return check_launch(who);
+  }
+  KP_LAUNCH_SPAN(first, false, emb_sort_chunks<false>, dim3((unsigned)g1), dim3(kSortThreads), 0, s, a, Z.s1);
+  const int st = check_launch(who);
+  if (st != KP_OK) return st;
+  hipLaunchKernelGGL(emb_rank, dim3((unsigned)g2), dim3(kThreads), 0, s, a, (int)rank_blocks, Z.s2);
+  return check_launch(who);
+}
+
 bool rows16(const void* p, int64_t stride) { return aligned16(p) && (stride & 7) == 0; }
 
 }  // namespace
@@ -935,8 +1133,7 @@ int kp_embedding_fwd_bf16(const void* table, int64_t V, int64_t D, int64_t table
   if (T == 0) return KP_OK;
   EmbFwdArgs a{static_cast<const uint16_t*>(table), V, D, table_row_stride, indices, index_bytes, T,
                static_cast<uint16_t*>(out), out_row_stride, error_flag};
-  const bool vec = (D % 8) == 0 && aligned16(table) && aligned16(out) && (table_row_stride % 8) == 0 &&
-                   (out_row_stride % 8) == 0;
+  const bool vec = D >= 8;  // any alignment: 16-byte accesses at 2-byte alignment
   const int64_t blocks_needed = ceil_div(T, kThreads / 64);
   hipStream_t s = as_stream(stream);
   if (vec) {  // one token per wave: the grid covers T
@@ -1008,52 +1205,37 @@ int kp_embedding_bwd_bf16(const void* grad, int64_t grad_row_stride, const void*
   a.bitmap = reinterpret_cast<uint32_t*>(ws + L.bitmap);
   a.pieces = reinterpret_cast<float*>(ws + L.pieces);
 
-  const bool vec = (D % 4) == 0 && aligned16(grad_table) &&
-                   (T == 0 || ((reinterpret_cast<uintptr_t>(grad) & 7u) == 0 && grad_row_stride % 4 == 0));
+  const bool vec = D >= 4;  // any alignment
   hipStream_t s = as_stream(stream);
   const int64_t nq = ceil_div(D, kColStep);
   const int64_t row_bytes = D * (out_dtype == KP_DTYPE_BF16 ? 2 : 4);
   const int64_t nwin_blocks = L.nwin * nq;
-  const int64_t total_keys = L.nchunks * kChunk;
-  const int64_t rank_blocks = ceil_div(total_keys, kThreads);
-  const int comb_blocks = cu_count() * 4;
+  const bool combine = L.nwin > 1;  // a single window holds every run whole
+  const int comb_blocks = (int)(L.nwin * nq < cu_count() * 4 ? L.nwin * nq : cu_count() * 4);
   for (int64_t lo = 0; lo < V; lo += kMaxVocab) {
     const int64_t Vs = V - lo < kMaxVocab ? V - lo : kMaxVocab;  // this pass's slab [lo, lo + Vs)
     const bool first = lo == 0, last = lo + Vs >= V;
     a.id_lo = lo;
     a.V = Vs;
     a.out = static_cast<uint8_t*>(grad_table) + lo * row_bytes;
-    // Zero-fill shares, taken from the top of the slab down (high ids are
-    // the rarely touched ones under the usual frequency-ordered vocabularies):
-    // K1 [Vs - z1, Vs), K2 [Vs - z1 - z2, Vs - z1), K4 [r3, Vs - z1 - z2), K3 [0, r3).
-    const int64_t z1 = share_rows("KP_EMB_ZERO_MB_SORT", 128, row_bytes, Vs / 4);
-    const int64_t z2 = share_rows("KP_EMB_ZERO_MB_RANK", 128, row_bytes, Vs / 4);
-    const int64_t z4 = share_rows("KP_EMB_ZERO_MB_COMBINE", 96, row_bytes, Vs / 4);
-    const ZeroShare zs1{Vs - z1, Vs, 0};
-    const ZeroShare zs2{Vs - z1 - z2, Vs - z1, 0};
-    const ZeroShare zs4{Vs - z1 - z2 - z4, Vs - z1 - z2, 1};
-    const ZeroShare zs3{0, Vs - z1 - z2 - z4, 1};
-    const int64_t g1 = L.nchunks + z1 * nq, g2 = rank_blocks + z2 * nq, g3 = nwin_blocks + zs3.hi * nq,
-                  g4 = comb_blocks + z4 * nq;
-    if (g1 > 0x7fffffffLL || g2 > 0x7fffffffLL || g3 > 0x7fffffffLL || g4 > 0x7fffffffLL)
+    const ZeroShares Z = make_shares(Vs, row_bytes, ranked_in_sort(a), combine);
+    const int64_t g3 = nwin_blocks + zero_blocks(Z.s3), g4 = comb_blocks + zero_blocks(Z.s4);
+    if (g3 > 0x7fffffffLL || g4 > 0x7fffffffLL)
       return fail(KP_EUNSUPPORTED, "%s: V * D too large for one launch", who);
     // With the timing hook set, the events span the whole pipeline (the first
-    // K1's start to the last K4's end): its zero fill is spread over all four
-    // launches.
-    int st;
-    if (vec) KP_LAUNCH_SPAN(first, false, emb_sort_chunks<true>, dim3((unsigned)g1), dim3(kThreads), 0, s, a, zs1);
-    else KP_LAUNCH_SPAN(first, false, emb_sort_chunks<false>, dim3((unsigned)g1), dim3(kThreads), 0, s, a, zs1);
-    if ((st = check_launch(who)) != KP_OK) return st;
-    if (vec) hipLaunchKernelGGL(emb_rank<true>, dim3((unsigned)g2), dim3(kThreads), 0, s, a, (int)rank_blocks, zs2);
-    else hipLaunchKernelGGL(emb_rank<false>, dim3((unsigned)g2), dim3(kThreads), 0, s, a, (int)rank_blocks, zs2);
-    if ((st = check_launch(who)) != KP_OK) return st;
-    if (vec) hipLaunchKernelGGL(emb_dense<true>, dim3((unsigned)g3), dim3(kThreads), 0, s, a, nwin_blocks, zs3);
-    else hipLaunchKernelGGL(emb_dense<false>, dim3((unsigned)g3), dim3(kThreads), 0, s, a, nwin_blocks, zs3);
-    if ((st = check_launch(who)) != KP_OK) return st;
+    // launch's start to the last one's end): its zero fill is spread over them.
+    int st = launch_sort(who, a, Z, first, s);
+    if (st != KP_OK) return st;
     if (vec)
-      KP_LAUNCH_SPAN(false, last, emb_combine<true>, dim3((unsigned)g4), dim3(kThreads), 0, s, a, comb_blocks, zs4);
+      KP_LAUNCH_SPAN(false, last && !combine, emb_dense<true>, dim3((unsigned)g3), dim3(kThreads), 0, s, a, nwin_blocks, Z.s3);
     else
-      KP_LAUNCH_SPAN(false, last, emb_combine<false>, dim3((unsigned)g4), dim3(kThreads), 0, s, a, comb_blocks, zs4);
+      KP_LAUNCH_SPAN(false, last && !combine, emb_dense<false>, dim3((unsigned)g3), dim3(kThreads), 0, s, a, nwin_blocks, Z.s3);
+    if ((st = check_launch(who)) != KP_OK) return st;
+    if (!combine) continue;
+    if (vec)
+      KP_LAUNCH_SPAN(false, last, emb_combine<true>, dim3((unsigned)g4), dim3(kThreads), 0, s, a, comb_blocks, Z.s4);
+    else
+      KP_LAUNCH_SPAN(false, last, emb_combine<false>, dim3((unsigned)g4), dim3(kThreads), 0, s, a, comb_blocks, Z.s4);
     if ((st = check_launch(who)) != KP_OK) return st;
   }
   return KP_OK;
@@ -1171,34 +1353,23 @@ int kp_rmsnorm_embedding_bwd_bf16(const void* const* dy_terms, const int64_t* dy
   // rest of the untouched rows go to K3's zero blocks, launched with no
   // window blocks after the fused row pass (whose registers would hold zero
   // blocks sharing its launch to a few per CU).
-  const int64_t z1 = share_rows("KP_EMB_ZERO_MB_SORT", 128, row_bytes, V / 4);
-  const int64_t z2 = share_rows("KP_EMB_ZERO_MB_RANK", 128, row_bytes, V / 4);
-  const int64_t z4 = share_rows("KP_EMB_ZERO_MB_COMBINE", 96, row_bytes, V / 4);
-  const ZeroShare zs1{V - z1, V, 0};
-  const ZeroShare zs2{V - z1 - z2, V - z1, 0};
-  const ZeroShare zs4{V - z1 - z2 - z4, V - z1 - z2, 1};
-  const ZeroShare zs3{0, V - z1 - z2 - z4, 1};
-  const int64_t total_keys = L.nchunks * kChunk;
-  const int64_t rank_blocks = ceil_div(total_keys, kThreads);
-  const int comb_blocks = cu_count() * 4;
-  const int64_t g1 = L.nchunks + z1 * nq, g2 = rank_blocks + z2 * nq, g3 = zs3.hi * nq, g4 = comb_blocks + z4 * nq;
-  if (g1 > 0x7fffffffLL || g2 > 0x7fffffffLL || g3 > 0x7fffffffLL || g4 > 0x7fffffffLL)
+  const ZeroShares Z = make_shares(V, row_bytes, ranked_in_sort(e), true);
+  const int comb_blocks = (int)(L.nwin * nq < cu_count() * 4 ? L.nwin * nq : cu_count() * 4);
+  const int64_t g3 = zero_blocks(Z.s3), g4 = comb_blocks + zero_blocks(Z.s4);
+  if (g3 > 0x7fffffffLL || g4 > 0x7fffffffLL)
     return fail(KP_EUNSUPPORTED, "%s: V * N too large for one launch", who);
-  int st;
-  KP_LAUNCH_SPAN(true, false, emb_sort_chunks<true>, dim3((unsigned)g1), dim3(kThreads), 0, s, e, zs1);
-  if ((st = check_launch(who)) != KP_OK) return st;
-  hipLaunchKernelGGL(emb_rank<true>, dim3((unsigned)g2), dim3(kThreads), 0, s, e, (int)rank_blocks, zs2);
-  if ((st = check_launch(who)) != KP_OK) return st;
+  int st = launch_sort(who, e, Z, true, s);
+  if (st != KP_OK) return st;
   const int64_t nblocks = CL.nwin + CL.nb2;  // window blocks, then norm-only blocks
   if (nblocks > 0) {
     hipLaunchKernelGGL(kern, dim3((unsigned)nblocks), dim3(nw * 64), 0, s, a, e, c);
     if ((st = check_launch(who)) != KP_OK) return st;
   }
   if (g3 > 0) {
-    hipLaunchKernelGGL(emb_dense<true>, dim3((unsigned)g3), dim3(kThreads), 0, s, e, (int64_t)0, zs3);
+    hipLaunchKernelGGL(emb_dense<true>, dim3((unsigned)g3), dim3(kThreads), 0, s, e, (int64_t)0, Z.s3);
     if ((st = check_launch(who)) != KP_OK) return st;
   }
-  KP_LAUNCH_SPAN(false, true, emb_combine<true>, dim3((unsigned)g4), dim3(kThreads), 0, s, e, comb_blocks, zs4);
+  if (g4 > 0) KP_LAUNCH_SPAN(false, true, emb_combine<true>, dim3((unsigned)g4), dim3(kThreads), 0, s, e, comb_blocks, Z.s4);
   if ((st = check_launch(who)) != KP_OK) return st;
   // The weight gradient: the partial rows in block order (none when M == 0:
   // zeros).
