@@ -3,9 +3,8 @@
 // One wave64 per (b, s) position handles every head of q and k at that
 // position, so the D/2 rotation angles are produced once per position and
 // shared by all H_q + H_k heads:
-//   - theta mode: inv_freq[f] = fp32(theta^(-2f/D)) (fp64 pow; for D = 128
-//     evaluated once per call on the host and passed in the kernel
-//     arguments, else by lane f in every wave), then per position
+//   - theta mode: inv_freq[f] = fp32(theta^(-2f/D)), evaluated in fp64 once
+//     per call on the host and passed in the kernel arguments, then per position
 //     a = fp32(fp32(p) * inv_freq[f]) and
 //     sincosf(a) (full-range OCML reduction, not a fast approximation).  The
 //     D/2 (cos, sin) pairs go to a per-wave LDS slot and are read back by the
@@ -45,16 +44,14 @@ struct RopeArgs {
   int pb;
   int64_t psb, pss;
   int pairing;
-  double theta;
   const float* freqs;  // complex64 table as float pairs
   int64_t frows, frs;  // rows, row stride in complex elements
   int conj;
   int32_t* err;
-  // theta mode with D = 128: inv_freq[f] = fp32(theta^(-2f/D)), evaluated
-  // once per call on the host (have_inv = 1) instead of in every wave (both
-  // kernels then read it, so their angles stay identical)
-  int have_inv;
-  float inv_freq[64];
+  // theta mode: inv_freq[f] = fp32(theta^(-2f/D)), evaluated once per call on
+  // the host instead of in every wave (every kernel reads it, so their angles
+  // stay identical)
+  float inv_freq[kMaxHalf];
 };
 
 // Output element offset o gets 8 values (16-byte bf16 / 32-byte fp32) or 1 value.
@@ -65,7 +62,17 @@ __device__ __forceinline__ void store8p(void* out, int out_f32, int64_t o, const
     st16_stream(static_cast<uint16_t*>(out) + o, pack8(v));
   }
 }
-__device__ __forceinline__ void store8(const RopeTensor& T, int64_t o, const float* v) { store8p(T.out, T.out_f32, o, v); }
+// The same at any element alignment.
+__device__ __forceinline__ void store8u(void* out, int out_f32, int64_t o, const float* v) {
+  if (out_f32) {
+    typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+    float* p = static_cast<float*>(out) + o;
+    *reinterpret_cast<f32x4_u*>(p) = f32x4{v[0], v[1], v[2], v[3]};
+    *reinterpret_cast<f32x4_u*>(p + 4) = f32x4{v[4], v[5], v[6], v[7]};
+  } else {
+    st16u_stream(static_cast<uint16_t*>(out) + o, pack8(v));
+  }
+}
 __device__ __forceinline__ void store1(const RopeTensor& T, int64_t o, float v) {
   if (T.out_f32) static_cast<float*>(T.out)[o] = v;
   else static_cast<uint16_t*>(T.out)[o] = f_to_bf(v);
@@ -80,26 +87,22 @@ __device__ __forceinline__ void rot(float a, float b, float c, float s, float& o
   ob = __builtin_fmaf(b, c, a * s);
 }
 
-// TABLE is a template parameter so that each instantiation reads its angles
-// from exactly one address space (global table or LDS slot); a runtime choice
-// lets the compiler merge both into one flat load.
-template <bool VEC, bool TABLE>
-__global__ __launch_bounds__(kThreads) void rope_kernel(RopeArgs a) {
+// D whose halves (rotate-half) or rows (interleaved) are no whole chunks: one
+// wave per (b, s) position, one rotation pair per lane and step.  TABLE is a
+// template parameter so that each instantiation reads its angles from exactly
+// one address space (global table or LDS slot); a runtime choice lets the
+// compiler merge both into one flat load.
+template <bool TABLE>
+__global__ __launch_bounds__(kThreads) void rope_scalar(RopeArgs a) {
   __shared__ float cs[kWavesPerBlock][2][kMaxHalf];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t half = a.D / 2;
-  constexpr bool table = TABLE;
 
   // inv_freq[f] for f = lane + 64k (theta mode), kept in registers.
   float inv[kMaxHalf / 64];
 #pragma unroll
-  for (int k = 0; k < kMaxHalf / 64; ++k) {
-    const int f = lane + 64 * k;
-    inv[k] = (!table && f < half)
-                 ? (a.have_inv ? a.inv_freq[f & 63] : (float)pow(a.theta, -(double)(2 * f) / (double)a.D))
-                 : 0.f;
-  }
+  for (int k = 0; k < kMaxHalf / 64; ++k) inv[k] = TABLE ? 0.f : a.inv_freq[lane + 64 * k];
 
   const int64_t npos = a.B * a.S;
   const int64_t w0 = (int64_t)blockIdx.x * kWavesPerBlock + wave;
@@ -108,9 +111,6 @@ __global__ __launch_bounds__(kThreads) void rope_kernel(RopeArgs a) {
   // The (cos, sin) slot is indexed through the __shared__ array itself (never
   // through a generic pointer) so reads stay ds_read; the workgroup-scope
   // fences around the wave barrier make the other lanes' ds_writes visible.
-#define COSV(f) cs[wave][0][f]
-#define SINV(f) cs[wave][1][f]
-
   for (int64_t ps = w0; ps < npos; ps += nw) {
     const int64_t b = ps / a.S, s = ps % a.S;
     int64_t p = s;
@@ -130,8 +130,8 @@ __global__ __launch_bounds__(kThreads) void rope_kernel(RopeArgs a) {
         if (f < half) {
           float sn, c;
           sincosf(pf * inv[k], &sn, &c);
-          COSV(f) = c;
-          SINV(f) = sn;
+          cs[wave][0][f] = c;
+          cs[wave][1][f] = sn;
         }
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -143,80 +143,25 @@ __global__ __launch_bounds__(kThreads) void rope_kernel(RopeArgs a) {
       const RopeTensor& T = a.t[ti];
       const uint16_t* xb = T.x + b * T.xs[0] + s * T.xs[1];
       const int64_t ob = b * T.os[0] + s * T.os[1];  // output element offset of this position
-      if constexpr (VEC) {
-        if (a.pairing == KP_ROPE_HALF) {
-          const int64_t nch = half / 8;  // chunks per half
-          for (int64_t u = lane; u < T.H * nch; u += 64) {
-            const int64_t h = u / nch, c = u % nch;
-            const uint16_t* xp = xb + h * T.xs[2] + c * 8;
-            const int64_t oo = ob + h * T.os[2] + c * 8;
-            float x1[8], x2[8], o1[8], o2[8];
-            unpack8(ld16_stream(xp), x1);
-            unpack8(ld16_stream(xp + half), x2);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              const int64_t f = c * 8 + e;
-              float cv, sv;
-              if constexpr (TABLE) {
-                cv = frow[2 * f];
-                sv = frow[2 * f + 1];
-              } else {
-                cv = COSV(f);
-                sv = SINV(f);
-              }
-              rot(x1[e], x2[e], cv, sgn * sv, o1[e], o2[e]);
-              if (!ok) o1[e] = o2[e] = 0.f;
-            }
-            store8(T, oo, o1);
-            store8(T, oo + half, o2);
-          }
+      for (int64_t u = lane; u < T.H * half; u += 64) {
+        const int64_t h = u / half, f = u % half;
+        const int64_t ia = a.pairing == KP_ROPE_HALF ? f : 2 * f;
+        const int64_t ib = a.pairing == KP_ROPE_HALF ? f + half : 2 * f + 1;
+        const uint16_t* xp = xb + h * T.xs[2];
+        const int64_t oo = ob + h * T.os[2];
+        float cv, sv;
+        if constexpr (TABLE) {
+          cv = frow[2 * f];
+          sv = frow[2 * f + 1];
         } else {
-          const int64_t nch = a.D / 8;  // chunks per head, 4 pairs each
-          for (int64_t u = lane; u < T.H * nch; u += 64) {
-            const int64_t h = u / nch, c = u % nch;
-            const uint16_t* xp = xb + h * T.xs[2] + c * 8;
-            const int64_t oo = ob + h * T.os[2] + c * 8;
-            float xv[8], o[8];
-            unpack8(ld16_stream(xp), xv);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const int64_t f = c * 4 + q;
-              float cv, sv;
-              if constexpr (TABLE) {
-                cv = frow[2 * f];
-                sv = frow[2 * f + 1];
-              } else {
-                cv = COSV(f);
-                sv = SINV(f);
-              }
-              rot(xv[2 * q], xv[2 * q + 1], cv, sgn * sv, o[2 * q], o[2 * q + 1]);
-              if (!ok) o[2 * q] = o[2 * q + 1] = 0.f;
-            }
-            store8(T, oo, o);
-          }
+          cv = cs[wave][0][f];
+          sv = cs[wave][1][f];
         }
-      } else {
-        // Scalar path: any alignment / stride, one rotation pair per step.
-        for (int64_t u = lane; u < T.H * half; u += 64) {
-          const int64_t h = u / half, f = u % half;
-          const int64_t ia = a.pairing == KP_ROPE_HALF ? f : 2 * f;
-          const int64_t ib = a.pairing == KP_ROPE_HALF ? f + half : 2 * f + 1;
-          const uint16_t* xp = xb + h * T.xs[2];
-          const int64_t oo = ob + h * T.os[2];
-          float cv, sv;
-          if constexpr (TABLE) {
-            cv = frow[2 * f];
-            sv = frow[2 * f + 1];
-          } else {
-            cv = COSV(f);
-            sv = SINV(f);
-          }
-          float oa, obv;
-          rot(bf_to_f(xp[ia]), bf_to_f(xp[ib]), cv, sgn * sv, oa, obv);
-          if (!ok) oa = obv = 0.f;
-          store1(T, oo + ia, oa);
-          store1(T, oo + ib, obv);
-        }
+        float oa, obv;
+        rot(bf_to_f(xp[ia]), bf_to_f(xp[ib]), cv, sgn * sv, oa, obv);
+        if (!ok) oa = obv = 0.f;
+        store1(T, oo + ia, oa);
+        store1(T, oo + ib, obv);
       }
     }
     if constexpr (!TABLE) {
@@ -228,8 +173,145 @@ __global__ __launch_bounds__(kThreads) void rope_kernel(RopeArgs a) {
   }
 }
 
-#undef COSV
-#undef SINV
+// ------------------------------------------------------------ wave path
+// Any D of whole chunks, any strides and alignment: one wave per (b, s)
+// position, every head of both tensors.  A unit is one 16-byte chunk of a
+// head; lane l takes units l, l + 64, ..., UPL of them requested together,
+// `step` units (whole heads) a round.
+// Rotate-half reads a chunk's partner (D/2 further or back) beside it: every
+// line is read by two lanes, the second time from cache, and a wave stores
+// whole consecutive chunks.  With the pair as the unit, a row's two halves
+// were loaded and stored as separate half lines: [4, 4096, 32 + 8, 64]
+// 37.4 us, so 27.0 us (6.2 TB/s), [4, 4096, 16 + 4, 96] 34.7 and 20.9 us.
+// The position is wave-uniform, so a unit's address is one multiply-add from
+// a scalar base.  The wave's angles are made while its first loads are in
+// flight -- sincosf in theta mode, the table's row (rotate-half) -- and go
+// through its LDS slot with the conjugate's sign; interleaved table mode
+// reads a chunk's 4 angles straight from the row.  Arithmetic, rounding and
+// angles are those of rope_scalar.  Against the loop of one unit at a time
+// with 64-bit divisions that these widths ran before: [3, 1009, 24 + 8, 64]
+// interleaved table 8.1 -> 6.8 us, [4, 4096, 32 + 8, 64] rotate-half 38.1 ->
+// 27.0 us, [4, 4096, 16 + 4, 80] interleaved 25.8 -> 18.1 us.
+template <int PAIRING, bool TABLE, int UPL>
+__global__ __launch_bounds__(kThreads) void rope_wave(RopeArgs a, Div32 by_c, Div32 by_s, uint32_t step) {
+  constexpr bool kHalf = PAIRING == KP_ROPE_HALF;
+  constexpr int FPU = kHalf ? 8 : 4;  // angles per unit
+  constexpr bool kStage = !TABLE || kHalf;
+  __shared__ float cs[kStage ? kWavesPerBlock : 1][2][kStage ? kMaxHalf : 1];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t ps = (uint32_t)blockIdx.x * kWavesPerBlock + wave;
+  if (ps >= (uint32_t)(a.B * a.S)) return;  // wave-uniform; only wave barriers follow
+  const uint32_t b = div32(ps, by_s), s = ps - b * by_s.d;
+  const int half = (int)(a.D / 2);
+  const RopeTensor &T0 = a.t[0], &T1 = a.t[a.nt > 1 ? 1 : 0];
+  const uint32_t U0 = (uint32_t)T0.H * by_c.d, U = U0 + (a.nt > 1 ? (uint32_t)T1.H * by_c.d : 0);
+  const uint16_t* xb0 = T0.x + b * T0.xs[0] + s * T0.xs[1];
+  const uint16_t* xb1 = T1.x + b * T1.xs[0] + s * T1.xs[1];
+  // wave-uniform output fields (see rope_fast_body)
+  const int64_t ob0 = uniform64(b * T0.os[0] + s * T0.os[1]), ob1 = uniform64(b * T1.os[0] + s * T1.os[1]);
+  const int64_t hs0 = uniform64(T0.os[2]), hs1 = uniform64(T1.os[2]);
+  char* const out0 = static_cast<char*>(T0.out);
+  const int64_t dout = uniform64(static_cast<char*>(T1.out) - out0);
+  const int f0 = __builtin_amdgcn_readfirstlane(T0.out_f32), f1 = __builtin_amdgcn_readfirstlane(T1.out_f32);
+  // The position id and the lane's first inverse frequency are requested before
+  // the data: loads complete in order, so waiting for them is not waiting for
+  // the data, and the angle work overlaps it.
+  int64_t p = s;
+  if (a.pos) p = a.pb == 8 ? static_cast<const int64_t*>(a.pos)[b * a.psb + s * a.pss]
+                           : (int64_t) static_cast<const int32_t*>(a.pos)[b * a.psb + s * a.pss];
+  const float inv0 = TABLE ? 0.f : a.inv_freq[lane];
+  __builtin_amdgcn_sched_barrier(0);
+  bool ok = true;
+  const float* frow = a.freqs;
+  const float sgn = a.conj ? -1.f : 1.f;
+  for (uint32_t base = 0; base < U; base += step) {
+    u32x4 v1[UPL], v2[UPL];
+    uint32_t hh[UPL], ch[UPL];
+#pragma unroll
+    for (int j = 0; j < UPL; ++j) {
+      uint32_t u = base + lane + 64 * j;
+      u = u < U ? u : U - 1;  // past the end: the last unit again, not stored
+      const bool second = u >= U0;
+      const uint32_t ul = second ? u - U0 : u;
+      hh[j] = div32(ul, by_c);
+      ch[j] = ul - hh[j] * by_c.d;
+      const uint16_t* xp = (second ? xb1 + hh[j] * T1.xs[2] : xb0 + hh[j] * T0.xs[2]) + ch[j] * 8;
+      v1[j] = ld16u(xp);
+      if constexpr (kHalf) v2[j] = ld16u(ch[j] * 16 < (uint32_t)a.D ? xp + half : xp - half);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (base == 0) {
+      if constexpr (TABLE) {
+        ok = p >= 0 && p < a.frows;  // an out-of-range id reads row 0: its outputs are zeroed
+        if (!ok && lane == 0 && a.err) *a.err = 1;
+        frow = a.freqs + 2 * ((ok ? p : 0) * a.frs);
+      }
+      if constexpr (kStage) {
+        for (int f = lane; f < half; f += 64) {
+          float sn, cn;
+          if constexpr (TABLE) {
+            cn = frow[2 * f];
+            sn = frow[2 * f + 1];
+          } else {
+            sincosf((float)p * (f < 64 ? inv0 : a.inv_freq[f]), &sn, &cn);
+          }
+          cs[wave][0][f] = cn;
+          cs[wave][1][f] = sgn * sn;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+      }
+    }
+    if constexpr (kHalf) {
+      // every load of the batch has arrived before its first store: a chunk and
+      // its partner are in one batch, so the rotation may be in place
+#pragma unroll
+      for (int j = 0; j < UPL; ++j) asm volatile("" : "+v"(v1[j]), "+v"(v2[j]));
+    }
+#pragma unroll
+    for (int j = 0; j < UPL; ++j) {
+      const uint32_t u = base + lane + 64 * j;
+      if (lane + 64 * j >= step || u >= U) continue;
+      const bool second = u >= U0;
+      const int64_t oo = (second ? ob1 + hh[j] * hs1 : ob0 + hh[j] * hs0) + ch[j] * 8;
+      void* out = out0 + (second ? dout : 0);
+      const int f32 = second ? f1 : f0;
+      const bool lower = ch[j] * 16 < (uint32_t)a.D;
+      const int fb = kHalf ? (int)(lower ? ch[j] * 8 : ch[j] * 8 - half) : (int)ch[j] * 4;
+      float cv[FPU], sv[FPU];
+#pragma unroll
+      for (int e = 0; e < FPU; ++e) {
+        if constexpr (kStage) {
+          cv[e] = cs[wave][0][fb + e];
+          sv[e] = cs[wave][1][fb + e];
+        } else {
+          cv[e] = frow[2 * (fb + e)];
+          sv[e] = sgn * frow[2 * (fb + e) + 1];
+        }
+      }
+      float x1[8], o1[8];
+      unpack8(v1[j], x1);
+      if constexpr (kHalf) {
+        float x2[8];
+        unpack8(v2[j], x2);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          o1[e] = __builtin_fmaf(x1[e], cv[e], x2[e] * (lower ? -sv[e] : sv[e]));
+          if (!ok) o1[e] = 0.f;
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          rot(x1[2 * q], x1[2 * q + 1], cv[q], sv[q], o1[2 * q], o1[2 * q + 1]);
+          if (!ok) o1[2 * q] = o1[2 * q + 1] = 0.f;
+        }
+      }
+      store8u(out, f32, oo, o1);
+    }
+  }
+}
 
 // ------------------------------------------------------------ fast path
 // D = 128 with 16-byte aligned rows (every reference fragment and the
@@ -244,7 +326,7 @@ __global__ __launch_bounds__(kThreads) void rope_kernel(RopeArgs a) {
 // head) and its 8 (or 4) rotation angles serve every unit it holds.  Units
 // past the end re-read the last unit (same lines, no predicated loads: see
 // the row kernels of kp_rmsnorm.hip) and store nothing.  Arithmetic, rounding
-// and angles are those of rope_kernel, so both paths give identical bits.
+// and angles are those of rope_scalar, so both paths give identical bits.
 constexpr int kFastD = 128;
 constexpr int kFastMaxLoads = 16;
 
@@ -302,7 +384,7 @@ __device__ __forceinline__ void rope_fast_body(const RopeArgs& a) {
     }
   } else {
     // lane f < D/2 produces angle f: fp32(fp32(p) * fp32(theta^(-2f/D)))
-    const float inv = a.have_inv ? a.inv_freq[lane] : (float)pow(a.theta, -(double)(2 * lane) / (double)kFastD);
+    const float inv = a.inv_freq[lane];
     float sn, cn;
     sincosf((float)p * inv, &sn, &cn);
     cs[wave][0][lane] = cn;
@@ -650,7 +732,7 @@ bool tile_ok(const RopeArgs& a, bool table) {
     const char* e = getenv("KP_ROPE_TILE");
     return e == nullptr || atoi(e) != 0;
   }();
-  if (!enabled || a.D != kFastD || (!table && !a.have_inv)) return false;
+  if (!enabled || a.D != kFastD) return false;
   if (table && (!aligned16(a.freqs) || (a.frs & 1) != 0)) return false;
   const int64_t npos = a.B * a.S;
   if (npos <= 0 || npos > INT32_MAX) return false;
@@ -688,7 +770,7 @@ RopeKernel fast_for_upl(int upl) {
   return nullptr;
 }
 
-// The fast kernel for this call, or nullptr (then rope_kernel runs).
+// The fast kernel for this call, or nullptr (then rope_wave runs).
 RopeKernel pick_fast(const RopeArgs& a, int pairing, bool table) {
   if (a.D != kFastD) return nullptr;
   if (table && (!aligned16(a.freqs) || (a.frs & 1) != 0)) return nullptr;
@@ -706,6 +788,50 @@ RopeKernel pick_fast(const RopeArgs& a, int pairing, bool table) {
     }
   if (half) return table ? fast_for_upl<KP_ROPE_HALF, true>((int)upl) : fast_for_upl<KP_ROPE_HALF, false>((int)upl);
   return table ? fast_for_upl<KP_ROPE_INTERLEAVED, true>((int)upl) : fast_for_upl<KP_ROPE_INTERLEAVED, false>((int)upl);
+}
+
+typedef void (*WaveKernel)(RopeArgs, Div32, Div32, uint32_t);
+
+template <int PAIRING, bool TABLE>
+WaveKernel wave_for_upl(int64_t upl) {
+  switch (upl) {
+    case 1: return rope_wave<PAIRING, TABLE, 1>;
+    case 2: return rope_wave<PAIRING, TABLE, 2>;
+    case 3: return rope_wave<PAIRING, TABLE, 3>;
+  }
+  return rope_wave<PAIRING, TABLE, 4>;
+}
+
+// The wave kernel for this call, or nullptr (D of no whole chunks, or more
+// positions or units than 32-bit indexes hold: then rope_scalar runs).
+WaveKernel pick_wave(const RopeArgs& a, int pairing, bool table, Div32* by_c, Div32* by_s, uint32_t* step) {
+  const bool half = pairing == KP_ROPE_HALF;
+  if (a.D % (half ? 16 : 8) != 0) return nullptr;
+  const int64_t cph = a.D / 8, H = a.t[0].H + (a.nt > 1 ? a.t[1].H : 0);
+  if (H <= 0 || H > (INT32_MAX - 4096) / cph || a.B * a.S > INT32_MAX - 4096) return nullptr;
+  *by_c = make_div32((uint32_t)cph);
+  *by_s = make_div32((uint32_t)a.S);
+  // Units in flight per lane: all of a position's while they are few; two in
+  // interleaved form, where more registers cost more than they hide
+  // ([4, 4096, 32 + 8, 64] table 28.8 us with two, 30.3 with three).
+  int64_t upl = ceil_div(H * cph, 64);
+  const int64_t most = half ? 4 : 2;
+  if (upl > most) upl = most;
+  *step = (uint32_t)(64 * upl / cph * cph);  // whole heads (a head is at most 64 chunks)
+  if (half) return table ? wave_for_upl<KP_ROPE_HALF, true>(upl) : wave_for_upl<KP_ROPE_HALF, false>(upl);
+  return table ? wave_for_upl<KP_ROPE_INTERLEAVED, true>(upl) : wave_for_upl<KP_ROPE_INTERLEAVED, false>(upl);
+}
+
+// inv[f] = fp32(theta^(-2f/D)), f < D / 2, as products of 16 + D / 32 powers:
+// each within a couple of fp64 roundings, far below fp32's.
+void fill_inv_freq(double theta, int64_t D, float* inv) {
+  double lo[16];
+  for (int i = 0; i < 16; ++i) lo[i] = pow(theta, -(double)(2 * i) / (double)D);
+  double hi = 1.0;
+  for (int f = 0; f < (int)(D / 2); ++f) {
+    if ((f & 15) == 0) hi = pow(theta, -(double)(2 * f) / (double)D);
+    inv[f] = (float)(hi * lo[f & 15]);
+  }
 }
 
 bool tensor_vec_ok(const RopeTensor& t, int64_t D, int pairing) {
@@ -762,16 +888,12 @@ static int rope_impl(const char* who, const void* x0, void* out0, int64_t H0, co
   a.psb = pos_stride_b;
   a.pss = pos_stride_s;
   a.pairing = pairing;
-  a.theta = theta;
   a.freqs = freqs_cis;
   a.frows = freq_rows;
   a.frs = freq_row_stride;
   a.conj = conj ? 1 : 0;
   a.err = error_flag;
-  if (freqs_cis == nullptr && D == kFastD) {  // the fast kernel's angles: one evaluation per call
-    a.have_inv = 1;
-    for (int f = 0; f < kFastD / 2; ++f) a.inv_freq[f] = (float)pow(theta, -(double)(2 * f) / (double)kFastD);
-  }
+  if (freqs_cis == nullptr) fill_inv_freq(theta, D, a.inv_freq);
   const int64_t npos = B * S;
   if (npos == 0) return KP_OK;
 
@@ -816,19 +938,22 @@ static int rope_impl(const char* who, const void* x0, void* out0, int64_t H0, co
       if (a.nt > 1) a.t[1].out = out1_copy;
     }
     const RopeKernel fk = vec ? pick_fast(a, pairing, freqs_cis != nullptr) : nullptr;
+    const bool tab = freqs_cis != nullptr;
+    hipStream_t st_ = as_stream(stream);
+    Div32 by_c{}, by_s{};
+    uint32_t step = 0;
+    const WaveKernel wk = fk == nullptr ? pick_wave(a, pairing, tab, &by_c, &by_s, &step) : nullptr;
     if (fk != nullptr && blocks_needed <= INT32_MAX) {
       void* args[] = {&a};
-      launch_dominant_raw(reinterpret_cast<const void*>(fk), dim3((unsigned)blocks_needed), dim3(kThreads), args, 0,
-                          as_stream(stream));
+      launch_dominant_raw(reinterpret_cast<const void*>(fk), dim3((unsigned)blocks_needed), dim3(kThreads), args, 0, st_);
+    } else if (wk != nullptr) {
+      void* args[] = {&a, &by_c, &by_s, &step};
+      launch_dominant_raw(reinterpret_cast<const void*>(wk), dim3((unsigned)blocks_needed), dim3(kThreads), args, 0, st_);
     } else {
       const int64_t cap = (int64_t)cu_count() * 16;
       const int grid = (int)(blocks_needed < cap ? blocks_needed : cap);
-      hipStream_t s = as_stream(stream);
-      const bool tab = freqs_cis != nullptr;
-      if (vec && tab) KP_LAUNCH_DOMINANT((rope_kernel<true, true>), dim3(grid), dim3(kThreads), 0, s, a);
-      else if (vec) KP_LAUNCH_DOMINANT((rope_kernel<true, false>), dim3(grid), dim3(kThreads), 0, s, a);
-      else if (tab) KP_LAUNCH_DOMINANT((rope_kernel<false, true>), dim3(grid), dim3(kThreads), 0, s, a);
-      else KP_LAUNCH_DOMINANT((rope_kernel<false, false>), dim3(grid), dim3(kThreads), 0, s, a);
+      if (tab) KP_LAUNCH_DOMINANT(rope_scalar<true>, dim3(grid), dim3(kThreads), 0, st_, a);
+      else KP_LAUNCH_DOMINANT(rope_scalar<false>, dim3(grid), dim3(kThreads), 0, st_, a);
     }
     const int st = check_launch(who);
     if (st != KP_OK) return st;
