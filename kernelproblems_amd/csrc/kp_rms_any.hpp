@@ -22,7 +22,7 @@
 // of the tensor-level entry points, against the scalar one-block-per-row
 // kernels that these shapes took before (2-byte accesses, every row read
 // twice, the weight-gradient partials updated in memory):
-//   add + norm forward [3001, 2880]        35.9 -> 13.7 us (5.1 TB/s)
+//   add + norm forward [3001, 2880]        35.9 -> 12.3 us (5.6 TB/s)
 //   forward + backward [65536, 128]       275   -> 19.7 us (two row kernels and the finalize, 84 MB)
 //   forward + backward of odd widths      8.9x at 90 us
 #pragma once
@@ -163,6 +163,90 @@ __global__ __launch_bounds__(kThreads) void rms_fwd_any(RmsFwdArgs a) {
       }
     }
     if (a.rstd != nullptr && part == 0 && sub == 0) a.rstd[row] = r;
+  }
+}
+
+// The same for rows of middling width: persistent 4-wave blocks walking row
+// groups grid-stride with the next group's loads in flight (two named register
+// slots, unrolled two steps, as in rms_fwd_vec), the weight loaded once.
+template <int VPL, int WPR, int NX>
+__global__ __launch_bounds__(kThreads) void rms_fwd_any_loop(RmsFwdArgs a) {
+  constexpr int RB = 4 / WPR;
+  __shared__ float red[2][4];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int part = wave % WPR, rloc = wave / WPR;
+  const AnyCols<64, VPL, WPR> cols(part, lane, (int)a.N);
+  u32x4 wv[VPL];
+  any_weight<64, VPL, WPR>(wv, a.w, a.w_seg_len, a.w_seg_stride, cols, a.N);
+  int it = 0;
+  auto load = [&](RawRow<VPL, NX>& s, int64_t row) {
+    row = clamp_row(row, a.M);
+#pragma unroll
+    for (int t = 0; t < NX; ++t) {
+      const uint16_t* p = a.x[t] + row * a.xs[t];
+#pragma unroll
+      for (int i = 0; i < VPL; ++i) s.v[t][i] = ld16u_stream(p + cols.start[i]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto proc = [&](const RawRow<VPL, NX>& s, int64_t row) {
+    u32x4 hv[VPL];
+    sum_raw<VPL, NX>(hv, s);
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      float f[8];
+      unpack8(hv[i], f);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float v = (i < VPL - 1 || e >= cols.skip) ? f[e] : 0.f;
+        ss = fmaf(v, v, ss);
+      }
+    }
+    ss = wave_sum(ss);
+    if constexpr (WPR > 1) {
+      if (lane == 0) red[it & 1][wave] = ss;
+      __syncthreads();
+      float t = 0.f;
+#pragma unroll
+      for (int q = 0; q < WPR; ++q) t += red[it & 1][rloc * WPR + q];
+      ss = t;
+      ++it;
+    }
+    if (row >= a.M) return;
+    const float r = 1.0f / sqrtf(ss / (float)a.N + a.eps);
+    uint16_t* yrow = a.y + row * a.ys;
+    uint16_t* hrow = NX > 1 && a.h != nullptr ? a.h + row * a.hs : nullptr;
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      float h[8], w[8], o[8];
+      unpack8(hv[i], h);
+      unpack8(wv[i], w);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = (h[e] * r) * w[e];
+      if (cols.on(i)) {
+        st16u_stream(yrow + cols.start[i], pack8(o));
+        if (hrow != nullptr) st16u_stream(hrow + cols.start[i], hv[i]);
+      }
+    }
+    if (a.rstd != nullptr && part == 0 && lane == 0) a.rstd[row] = r;
+  };
+  const int64_t G = gridDim.x, nb = block_trips(ceil_div_dev(a.M, RB), blockIdx.x, G);
+  RawRow<VPL, NX> s0, s1;
+  int64_t g = blockIdx.x, k = 0;
+  load(s0, g * RB + rloc);
+  for (; k + 2 < nb; k += 2, g += 2 * G) {
+    load(s1, (g + G) * RB + rloc);
+    proc(s0, g * RB + rloc);
+    load(s0, (g + 2 * G) * RB + rloc);
+    proc(s1, (g + G) * RB + rloc);
+  }
+  if (k + 1 < nb) {
+    load(s1, (g + G) * RB + rloc);
+    proc(s0, g * RB + rloc);
+    proc(s1, (g + G) * RB + rloc);
+  } else {
+    proc(s0, g * RB + rloc);
   }
 }
 
@@ -353,6 +437,7 @@ __global__ __launch_bounds__(kAnyWaves * 64) void rms_bwd_any(RmsBwdArgs a) {
 // Kernels for a shape and term counts, or nullptr (kp_rms_fwd_any.hip,
 // kp_rms_bwd_any_1.hip, kp_rms_bwd_any_2.hip).
 FwdKernel fwd_any_kernel(const AnyShape& s, int nx);
+FwdKernel fwd_any_loop_kernel(const AnyShape& s, int nx);
 BwdKernel bwd_any_kernel_short(const AnyShape& s, int nx, int ndy, bool res);
 BwdKernel bwd_any_kernel_wide(const AnyShape& s, int nx, int ndy, bool res);
 inline BwdKernel bwd_any_kernel(const AnyShape& s, int nx, int ndy, bool res) {

@@ -25,14 +25,18 @@ constexpr AnyTail any_tail(int c, int N) {
 }
 
 // Row shapes: every chunk index below VPL - 1 lies wholly inside the row, i.e.
-// (VPL - 1) * 8 * LPR * WPR <= N.  Forward (4-wave blocks): lanes per row, chunks per lane, waves
-// per row, rows in flight per lane group; backward (8-wave blocks) without
-// the last.
+// (VPL - 1) * 8 * LPR * WPR <= N.  Lanes per row, chunks per lane, waves per
+// row and rows in flight per lane group (one-shot forward); 4-wave blocks
+// forward, 8-wave blocks backward.
 struct AnyShape {
   int lpr, vpl, wpr, u;
 };
-// false: no shape (N outside [kAnyMinN, kAnyMaxN]).
-constexpr bool any_fwd_shape(int64_t N, AnyShape* s) {
+// One-shot forward of `rows` input rows (M times the terms).  false: no shape
+// (N outside [kAnyMinN, kAnyMaxN]).  Short rows take several per lane group
+// once that still leaves four blocks' input for each of cus CUs: [65536, 128]
+// 6.9 us with four and 7.1 with one, [32768, 128] of two terms 6.4 and 7.7,
+// but [16384, 128] 4.1 and 3.6, [2048, 500] 3.8 and 3.3.
+constexpr bool any_fwd_shape(int64_t rows, int64_t N, int cus, AnyShape* s) {
   if (N < kAnyMinN || N > kAnyMaxN) return false;
   if (N <= 64) *s = {8, 1, 1, 4};
   else if (N <= 128) *s = {16, 1, 1, 4};
@@ -41,6 +45,14 @@ constexpr bool any_fwd_shape(int64_t N, AnyShape* s) {
   else if (N <= 1024) *s = {64, 2, 1, 2};
   else if (N <= 2048) *s = {64, 2, 2, 1};
   else *s = {64, (int)((N + 2047) / 2048), 4, 1};
+  if (rows < (int64_t)4 * cus * (4 / s->wpr) * (64 / s->lpr) * s->u) s->u = 1;
+  return true;
+}
+// Persistent forward: one wave per row, or two, of at most 5 chunks per lane.
+constexpr bool any_loop_shape(int64_t N, AnyShape* s) {
+  if (N <= 1024 || N > 5120) return false;
+  const int wpr = N <= 2560 ? 1 : 2;
+  *s = {64, (int)((N + 512 * wpr - 1) / (512 * wpr)), wpr, 1};
   return true;
 }
 constexpr bool any_bwd_shape(int64_t N, AnyShape* s) {

@@ -319,8 +319,8 @@ size_t bwd_workspace_size(int64_t M, int64_t N) {
   const int64_t rows = M < blocks ? M : blocks;
   return (size_t)(rows * ceil_div(N, kPartChunk) * kPartChunk * (int64_t)sizeof(float));
 }
-// The fused forward + backward also keeps room for an fp32 rstd per row after
-// the partial rows (used only by its two-launch fallback).
+// The fused forward + backward's size has room for an fp32 rstd per row after
+// the partial rows, as callers have allocated it.
 size_t fwd_bwd_workspace_size(int64_t M, int64_t N) {
   if (M <= 0 || N <= 0) return 16;
   return ((bwd_workspace_size(M, N) + 255) & ~(size_t)255) + (size_t)M * sizeof(float);
@@ -371,8 +371,6 @@ BwdPlan plan_bwd(const void* const* dy_terms, const int64_t* dy_strides, int n_d
   return p;
 }
 
-size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
-
 // Bytes of the partial rows a plan writes.
 size_t partial_bytes(const BwdPlan& p, int64_t N) {
   return (size_t)p.blocks * (size_t)(ceil_div(N, kPartChunk) * kPartChunk) * sizeof(float);
@@ -381,9 +379,9 @@ size_t partial_bytes(const BwdPlan& p, int64_t N) {
 // The RMSNorm backward (fo == nullptr) and the fused forward + backward
 // (fo != nullptr: rstd is recomputed and y / h / rstd are written by the same
 // row pass).  Shapes or term combinations without a fused kernel run the
-// forward kernel and then the backward with the rstd it wrote (workspace
-// bytes past the partial rows hold it when the caller wants no rstd).  The
-// workspace must hold the partial rows the launch plan writes (the *_size
+// forward kernel and then the backward, which recomputes rstd: the rows'
+// layouts may differ, and so the last bit of a sum, and dx and dw are to be
+// those of the backward called without rstd.  The workspace must hold the partial rows the launch plan writes (the *_size
 // functions return an upper bound of that).
 int rms_bwd_impl(const char* who, const void* const* dy_terms, const int64_t* dy_strides, int n_dy,
                  const void* const* x_terms, const int64_t* x_strides, int n_x, const float* rstd, const void* weight,
@@ -410,9 +408,7 @@ int rms_bwd_impl(const char* who, const void* const* dy_terms, const int64_t* dy
   if (two_launch)
     plan = plan_bwd(dy_terms, dy_strides, n_dy, x_terms, x_strides, n_x, weight, w_seg_len, w_seg_stride,
                     dx_residual, dxr_stride, dx, dx_stride, want_dw, nullptr, M, N);
-  const size_t part = want_dw ? partial_bytes(plan, N) : 0;
-  const bool rstd_in_ws = two_launch && fo->rstd == nullptr;
-  const size_t need = rstd_in_ws ? align256(part) + (size_t)M * sizeof(float) : part;
+  const size_t need = want_dw ? partial_bytes(plan, N) : 0;
   if (need > 0 && (workspace == nullptr || workspace_bytes < need || !aligned16(workspace)))
     return fail(KP_EWORKSPACE, "%s: workspace needs %zu bytes, 16-byte aligned (got %zu)", who, need, workspace_bytes);
 
@@ -445,11 +441,9 @@ int rms_bwd_impl(const char* who, const void* const* dy_terms, const int64_t* dy
 
   if (M > 0) {
     if (two_launch) {
-      float* r = rstd_in_ws ? reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + align256(part)) : fo->rstd;
       st = kp_rmsnorm_fwd_bf16(x_terms, x_strides, n_x, weight, w_seg_len, w_seg_stride, n_x > 1 ? fo->h : nullptr,
-                               fo->hs, fo->y, fo->ys, r, M, N, eps, stream);
+                               fo->hs, fo->y, fo->ys, fo->rstd, M, N, eps, stream);
       if (st != KP_OK) return st;
-      a.rstd = r;
     } else if (fo != nullptr) {
       a.y = fo->y;
       a.ys = fo->ys;
@@ -581,6 +575,12 @@ int kp_rmsnorm_fwd_bf16(const void* const* x_terms, const int64_t* x_strides, in
   bool vec = pick_fwd(M, N, &vpl, &wpr) && rows_vec_ok(x_terms, x_strides, n_x) && aligned16(y) && (y_stride & 7) == 0;
   if (vec && h_out) vec = aligned16(h_out) && (h_stride & 7) == 0;
   if (vec && weight) vec = aligned16(weight) && (w_seg_len & 7) == 0 && (w_seg_stride & 7) == 0;
+  // A few wide rows: four waves per row from the kernels for any width, a block
+  // per row, finish sooner than a row's one or two waves, and without the
+  // large grid's starting pause (two terms, 16 rows: 4096 columns 4.0 -> 2.7
+  // us, 2560 3.1 -> 2.6, 8192 3.5 -> 3.1; 256 rows of 4096 5.1 -> 3.7, 1024
+  // rows 7.1 both).
+  vec = vec && !(M <= cu_count() && N > 2048);
   const FwdKernel fk = vec ? fwd_kernel(vpl, wpr, n_x) : nullptr;
   vec = vec && fk != nullptr;
   hipStream_t s = as_stream(stream);
@@ -599,8 +599,25 @@ int kp_rmsnorm_fwd_bf16(const void* const* x_terms, const int64_t* x_strides, in
     launch_dominant_raw(reinterpret_cast<const void*>(fk), dim3(grid), dim3(kThreads), args, 0, s);
     return check_launch(who);
   }
-  AnyShape as{};
-  const FwdKernel ak = any_fwd_shape(N, &as) ? fwd_any_kernel(as, n_x) : nullptr;
+  // Any width and alignment.  Rows of middling width, more of them than CUs,
+  // run the persistent loop (us, one-shot / loop: [3001, 2880] two terms 14.0 /
+  // 12.3, [4096, 4095] 15.8 / 13.8, [16384, 2881] two terms 79.8 / 72.5); few
+  // or short rows are as fast or faster with a block each ([2048, 1001] two
+  // terms 4.9 / 5.2), wider ones too ([8192, 5121] two terms 72.0 / 74.9), and
+  // so are rows on 16-byte addresses once the call's traffic is beyond the
+  // Infinity Cache ([8192, 5120] two terms 56.0 / 58.9).
+  AnyShape as{}, ls{};
+  const FwdKernel ak = any_fwd_shape(M * n_x, N, cu_count(), &as) ? fwd_any_kernel(as, n_x) : nullptr;
+  const bool streamed = (N & 7) == 0 && rows_vec_ok(x_terms, x_strides, n_x) &&
+                        M * N * 2 * (n_x + (n_x > 1 && h_out != nullptr ? 2 : 1)) > ((int64_t)160 << 20);
+  const FwdKernel lk = M > cu_count() && !streamed && any_loop_shape(N, &ls) ? fwd_any_loop_kernel(ls, n_x) : nullptr;
+  if (lk != nullptr) {
+    const int64_t lgroups = ceil_div(M, 4 / ls.wpr), cap = (int64_t)cu_count() * fwd_bpc((int64_t)n_x * ls.vpl * 1024);
+    void* args[] = {&a};
+    launch_dominant_raw(reinterpret_cast<const void*>(lk), dim3((unsigned)(lgroups < cap ? lgroups : cap)),
+                        dim3(kThreads), args, 0, s);
+    return check_launch(who);
+  }
   const int64_t groups = ak != nullptr ? ceil_div(M, (int64_t)(4 / as.wpr) * (64 / as.lpr) * as.u) : 0;
   if (ak != nullptr && groups <= INT32_MAX) {
     void* args[] = {&a};

@@ -34,8 +34,12 @@ int main() {
   AnyShape s{};
   for (int64_t N = -1; N <= kAnyMaxN + 9; ++N) {
     const bool in = N >= kAnyMinN && N <= kAnyMaxN;
-    if (any_fwd_shape(N, &s) != in) ++bad;
-    else if (in && (check((int)N, s) != 0 || 4 % s.wpr != 0)) ++bad, std::printf("forward N=%d\n", (int)N);
+    for (int64_t M : {(int64_t)1, (int64_t)1 << 20}) {
+      if (any_fwd_shape(M, N, 256, &s) != in) ++bad;
+      else if (in && (check((int)N, s) != 0 || 4 % s.wpr != 0 || s.u < 1)) ++bad, std::printf("forward N=%d\n", (int)N);
+    }
+    if (any_loop_shape(N, &s) != (N > 1024 && N <= 5120)) ++bad;
+    else if (N > 1024 && N <= 5120 && (check((int)N, s) != 0 || 4 % s.wpr != 0 || s.vpl > 5)) ++bad, std::printf("loop N=%d\n", (int)N);
     if (any_bwd_shape(N, &s) != in) ++bad;
     else if (in && (check((int)N, s) != 0 || kAnyWaves % s.wpr != 0)) ++bad, std::printf("backward N=%d\n", (int)N);
   }

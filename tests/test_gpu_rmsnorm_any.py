@@ -62,6 +62,23 @@ def test_widths(gpu, N, M, terms):
     assert torch.equal(again[0], dx) and torch.equal(again[1], dw)
 
 
+@pytest.mark.parametrize("M,N", [(131077, 33), (131077, 64), (66001, 128), (33000, 200), (17001, 500), (9001, 1000),
+                                 (40000, 2049), (20000, 4098)])
+def test_many_rows(gpu, M, N):
+    """Enough rows for several per lane group, and traffic beyond the persistent loop's."""
+    x = [_rand(gpu, i, M, N) for i in range(2)]
+    w = _rand(gpu, 7, N) * 0.02 + 1
+    h, y, rstd = kp.rms_norm(x, w, EPS, N, return_h=True)
+    assert torch.equal(h, x[0] + x[1])
+    r64 = (h.double().square().mean(-1) + EPS).rsqrt()
+    torch.testing.assert_close(rstd.view(-1).double(), r64, rtol=1e-6, atol=0)
+    rows = torch.arange(0, M, 97, device=gpu)
+    y64 = h[rows].double() * r64[rows, None] * w.double()
+    assert_bf16_close(to_u16(y[rows]), to_u16(y64.to(torch.bfloat16)), what="y", max_ulp=1, min_exact=0.99)
+    last = h[-1:].double() * r64[-1:, None] * w.double()
+    assert_bf16_close(to_u16(y[-1:]), to_u16(last.to(torch.bfloat16)), what="last row", max_ulp=1)
+
+
 @pytest.mark.parametrize("N", [128, 1000, 4096])
 def test_views_and_segments(gpu, N):
     """Rows starting 3 elements into a wider buffer, and a weight viewed as 8 rows of it."""
