@@ -1136,10 +1136,18 @@ int kp_embedding_fwd_bf16(const void* table, int64_t V, int64_t D, int64_t table
   const bool vec = D >= 8;  // any alignment: 16-byte accesses at 2-byte alignment
   const int64_t blocks_needed = ceil_div(T, kThreads / 64);
   hipStream_t s = as_stream(stream);
-  if (vec) {  // one token per wave: the grid covers T
-    if (blocks_needed > 0x7fffffff) return fail(KP_EUNSUPPORTED, "%s: T = %lld tokens exceeds one launch", who, (long long)T);
-    if (index_bytes == 8) KP_LAUNCH_DOMINANT(emb_fwd_vec<8>, dim3((unsigned)blocks_needed), dim3(kThreads), 0, s, a);
-    else KP_LAUNCH_DOMINANT(emb_fwd_vec<4>, dim3((unsigned)blocks_needed), dim3(kThreads), 0, s, a);
+  if (vec) {  // one token per wave: the grid covers T, a slab of tokens per launch
+    constexpr int64_t kSlab = max_blocks(kThreads) * (kThreads / 64);
+    for (int64_t t0 = 0; t0 < T; t0 += kSlab) {
+      a.T = T - t0 < kSlab ? T - t0 : kSlab;
+      a.idx = static_cast<const char*>(indices) + t0 * index_bytes;
+      a.out = static_cast<uint16_t*>(out) + t0 * out_row_stride;
+      const unsigned blocks = (unsigned)ceil_div(a.T, kThreads / 64);
+      if (index_bytes == 8) KP_LAUNCH_DOMINANT(emb_fwd_vec<8>, dim3(blocks), dim3(kThreads), 0, s, a);
+      else KP_LAUNCH_DOMINANT(emb_fwd_vec<4>, dim3(blocks), dim3(kThreads), 0, s, a);
+      const int st = check_launch(who);
+      if (st != KP_OK) return st;
+    }
   } else {
     const int64_t cap = (int64_t)cu_count() * 16;
     const int grid = (int)(blocks_needed < cap ? blocks_needed : cap);

@@ -38,6 +38,8 @@ void launch_dominant_raw(const void* fn, dim3 grid, dim3 block, void** args, siz
 int rms_dw_finalize_launch(const float* partial, int P, int64_t N, float* dw_f32, uint16_t* dw_bf16, int round_f32,
                            hipStream_t s, const char* who);
 
+// Blocks of one launch: a dispatch counts its work-items in 32 bits.
+constexpr int64_t max_blocks(int threads) { return 0xffffffffLL / threads; }
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }

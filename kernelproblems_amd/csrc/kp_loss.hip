@@ -838,19 +838,33 @@ int kp_cross_entropy_fwd_bwd_bf16(const void* logits, int64_t row_stride, int64_
     a.row_valid = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + (size_t)M * sizeof(double));
   }
   if (M > 0) {
-    // the targets' buffer descriptor is 32-bit
-    const FbPlan plan = M * target_bytes <= 0xffffffffLL ? fb_plan(V) : FbPlan{nullptr, 0, 0, false};
-    void* args[] = {&a};
-    if (plan.kernel != nullptr) {
-      const int64_t cus = cu_count(), groups = ceil_div(M, plan.rows);
-      const unsigned blocks = (unsigned)(plan.persistent && groups > cus ? cus : groups);
-      launch_dominant_raw(reinterpret_cast<const void*>(plan.kernel), dim3(blocks), dim3(plan.threads), args, 0, st);
-    } else {
-      launch_dominant_raw(reinterpret_cast<const void*>(xent_fwd_bwd_scalar), dim3((unsigned)M), dim3(kThreads), args,
-                          0, st);
+    // Rows in slabs of what one launch takes: its work-items and the targets'
+    // buffer descriptor are 32-bit.
+    const FbPlan plan = fb_plan(V);
+    const int64_t by_blocks = plan.kernel != nullptr ? max_blocks(plan.threads) * plan.rows : max_blocks(kThreads);
+    const int64_t slab = by_blocks < 0xffffffffLL / target_bytes ? by_blocks : 0xffffffffLL / target_bytes;
+    for (int64_t r0 = 0; r0 < M; r0 += slab) {
+      FbArgs b = a;
+      b.M = M - r0 < slab ? M - r0 : slab;
+      b.logits += r0 * row_stride;
+      b.out += r0 * out_row_stride;
+      b.targets = static_cast<const char*>(targets) + r0 * target_bytes;
+      if (want_loss) {
+        b.row_loss += r0;
+        b.row_valid += r0;
+      }
+      void* args[] = {&b};
+      if (plan.kernel != nullptr) {
+        const int64_t cus = cu_count(), groups = ceil_div(b.M, plan.rows);
+        const unsigned blocks = (unsigned)(plan.persistent && groups > cus ? cus : groups);
+        launch_dominant_raw(reinterpret_cast<const void*>(plan.kernel), dim3(blocks), dim3(plan.threads), args, 0, st);
+      } else {
+        launch_dominant_raw(reinterpret_cast<const void*>(xent_fwd_bwd_scalar), dim3((unsigned)b.M), dim3(kThreads),
+                            args, 0, st);
+      }
+      const int rc = check_launch(who);
+      if (rc != KP_OK) return rc;
     }
-    const int rc = check_launch(who);
-    if (rc != KP_OK) return rc;
   }
   if (!want_loss) return KP_OK;
   hipLaunchKernelGGL(xent_fwd_finish, dim3(1), dim3(kFinThreads), 0, st, a.row_loss, a.row_valid, M, (double)scale,

@@ -619,7 +619,7 @@ int kp_rmsnorm_fwd_bf16(const void* const* x_terms, const int64_t* x_strides, in
     return check_launch(who);
   }
   const int64_t groups = ak != nullptr ? ceil_div(M, (int64_t)(4 / as.wpr) * (64 / as.lpr) * as.u) : 0;
-  if (ak != nullptr && groups <= INT32_MAX) {
+  if (ak != nullptr && groups <= max_blocks(kThreads)) {
     void* args[] = {&a};
     launch_dominant_raw(reinterpret_cast<const void*>(ak), dim3((unsigned)groups), dim3(kThreads), args, 0, s);
   } else {

@@ -193,14 +193,15 @@ __global__ __launch_bounds__(kThreads) void rope_scalar(RopeArgs a) {
 // interleaved table 8.1 -> 6.8 us, [4, 4096, 32 + 8, 64] rotate-half 38.1 ->
 // 27.0 us, [4, 4096, 16 + 4, 80] interleaved 25.8 -> 18.1 us.
 template <int PAIRING, bool TABLE, int UPL>
-__global__ __launch_bounds__(kThreads) void rope_wave(RopeArgs a, Div32 by_c, Div32 by_s, uint32_t step) {
+__global__ __launch_bounds__(kThreads) void rope_wave(RopeArgs a, Div32 by_c, Div32 by_s, uint32_t step,
+                                                       uint32_t first) {
   constexpr bool kHalf = PAIRING == KP_ROPE_HALF;
   constexpr int FPU = kHalf ? 8 : 4;  // angles per unit
   constexpr bool kStage = !TABLE || kHalf;
   __shared__ float cs[kStage ? kWavesPerBlock : 1][2][kStage ? kMaxHalf : 1];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t ps = (uint32_t)blockIdx.x * kWavesPerBlock + wave;
+  const uint32_t ps = first + (uint32_t)blockIdx.x * kWavesPerBlock + wave;
   if (ps >= (uint32_t)(a.B * a.S)) return;  // wave-uniform; only wave barriers follow
   const uint32_t b = div32(ps, by_s), s = ps - b * by_s.d;
   const int half = (int)(a.D / 2);
@@ -790,7 +791,7 @@ RopeKernel pick_fast(const RopeArgs& a, int pairing, bool table) {
   return table ? fast_for_upl<KP_ROPE_INTERLEAVED, true>((int)upl) : fast_for_upl<KP_ROPE_INTERLEAVED, false>((int)upl);
 }
 
-typedef void (*WaveKernel)(RopeArgs, Div32, Div32, uint32_t);
+typedef void (*WaveKernel)(RopeArgs, Div32, Div32, uint32_t, uint32_t);
 
 template <int PAIRING, bool TABLE>
 WaveKernel wave_for_upl(int64_t upl) {
@@ -947,8 +948,13 @@ static int rope_impl(const char* who, const void* x0, void* out0, int64_t H0, co
       void* args[] = {&a};
       launch_dominant_raw(reinterpret_cast<const void*>(fk), dim3((unsigned)blocks_needed), dim3(kThreads), args, 0, st_);
     } else if (wk != nullptr) {
-      void* args[] = {&a, &by_c, &by_s, &step};
-      launch_dominant_raw(reinterpret_cast<const void*>(wk), dim3((unsigned)blocks_needed), dim3(kThreads), args, 0, st_);
+      // a position per wave: as many launches as it takes blocks
+      for (int64_t b0 = 0; b0 < blocks_needed; b0 += max_blocks(kThreads)) {
+        const int64_t nb = blocks_needed - b0 < max_blocks(kThreads) ? blocks_needed - b0 : max_blocks(kThreads);
+        uint32_t first = (uint32_t)(b0 * kWavesPerBlock);
+        void* args[] = {&a, &by_c, &by_s, &step, &first};
+        launch_dominant_raw(reinterpret_cast<const void*>(wk), dim3((unsigned)nb), dim3(kThreads), args, 0, st_);
+      }
     } else {
       const int64_t cap = (int64_t)cu_count() * 16;
       const int grid = (int)(blocks_needed < cap ? blocks_needed : cap);

@@ -241,13 +241,13 @@ __global__ __launch_bounds__(kThreads) void swiglu_fwd_bwd_scalar(ScalarArgs a) 
 // ------------------------------------------------------------------ host side
 // Validates and launches one pointwise op over nin inputs / nout outputs of an
 // [M, N] bf16 matrix (unit inner stride, row strides in elements).
-template <bool ROWS>
+template <int PER, bool ROWS>
 const void* vec_kernel(int op) {
   switch (op) {
-    case kFwd: return reinterpret_cast<const void*>(swiglu_vec<kFwd, 1, ROWS>);
-    case kBwd: return reinterpret_cast<const void*>(swiglu_vec<kBwd, 1, ROWS>);
-    case kSilu: return reinterpret_cast<const void*>(swiglu_vec<kSilu, 1, ROWS>);
-    default: return reinterpret_cast<const void*>(swiglu_vec<kFwdBwd, 1, ROWS>);
+    case kFwd: return reinterpret_cast<const void*>(swiglu_vec<kFwd, PER, ROWS>);
+    case kBwd: return reinterpret_cast<const void*>(swiglu_vec<kBwd, PER, ROWS>);
+    case kSilu: return reinterpret_cast<const void*>(swiglu_vec<kSilu, PER, ROWS>);
+    default: return reinterpret_cast<const void*>(swiglu_vec<kFwdBwd, PER, ROWS>);
   }
 }
 
@@ -301,13 +301,13 @@ int launch_pointwise(const char* who, int op, const void* const* in, const int64
     // [16, 14336] 4.2 / 7.2.  Only the flat backward's four reads and two
     // writes stream better four at a time once they are large: [2048, 14336]
     // 58.0 / 59.7, [3072, 14336] 88.1 / 88.0, [4096, 14336] 119.5 / 116.4,
-    // [8192, 14336] 240 / 229.
-    const int per = flat && op == kBwd && a.total >= (int64_t)6 << 20 ? 4 : 1;
+    // [8192, 14336] 240 / 229.  Flat arrays of more chunks than one launch has
+    // threads (68 GB each) take four as well.
+    const int64_t most = max_blocks(kThreads) * kThreads;
+    const int per = flat && ((op == kBwd && a.total >= (int64_t)6 << 20) || a.total > most) ? 4 : 1;
     const int64_t blocks = ceil_div(a.total, (int64_t)kThreads * per);
-    if (blocks > 0x7fffffffLL) return fail(KP_EUNSUPPORTED, "%s: too many blocks for one launch", who);
-    const void* fk = per == 4 ? reinterpret_cast<const void*>(swiglu_vec<kBwd, 4, false>)
-                     : flat   ? vec_kernel<false>(op)
-                              : vec_kernel<true>(op);
+    if (blocks > max_blocks(kThreads)) return fail(KP_EUNSUPPORTED, "%s: too many blocks for one launch", who);
+    const void* fk = per == 4 ? vec_kernel<4, false>(op) : flat ? vec_kernel<1, false>(op) : vec_kernel<1, true>(op);
     void* args[] = {&a};
     launch_dominant_raw(fk, dim3((unsigned)blocks), dim3(kThreads), args, 0, stream);
     return check_launch(who);
