@@ -301,10 +301,10 @@ int launch_pointwise(const char* who, int op, const void* const* in, const int64
     // [16, 14336] 4.2 / 7.2.  Only the flat backward's four reads and two
     // writes stream better four at a time once they are large: [2048, 14336]
     // 58.0 / 59.7, [3072, 14336] 88.1 / 88.0, [4096, 14336] 119.5 / 116.4,
-    // [8192, 14336] 240 / 229.  Flat arrays of more chunks than one launch has
+    // [8192, 14336] 240 / 229; and silu alone: [8192, 14336] 79.5 / 77.0.  Flat arrays of more chunks than one launch has
     // threads (68 GB each) take four as well.
     const int64_t most = max_blocks(kThreads) * kThreads;
-    const int per = flat && ((op == kBwd && a.total >= (int64_t)6 << 20) || a.total > most) ? 4 : 1;
+    const int per = flat && (((op == kBwd || op == kSilu) && a.total >= (int64_t)6 << 20) || a.total > most) ? 4 : 1;
     const int64_t blocks = ceil_div(a.total, (int64_t)kThreads * per);
     if (blocks > max_blocks(kThreads)) return fail(KP_EUNSUPPORTED, "%s: too many blocks for one launch", who);
     const void* fk = per == 4 ? vec_kernel<4, false>(op) : flat ? vec_kernel<1, false>(op) : vec_kernel<1, true>(op);
