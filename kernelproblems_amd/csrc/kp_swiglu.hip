@@ -25,6 +25,7 @@
 // kernel with the same arithmetic.
 #include "kp_common.hpp"
 #include "kp_internal.hpp"
+#include "kp_row_chunks.hpp"
 
 namespace kp {
 namespace {
@@ -135,7 +136,7 @@ struct VecArgs {
   uint16_t* out[3];
   int64_t in_rs[4], out_rs[3];  // row strides in elements (rows only)
   int64_t n;
-  int64_t total;  // chunks of all rows (below 2^31 for rows)
+  int64_t total;  // chunks of all rows (at most kMaxRowChunks for rows)
   Div32 cpr;      // rows only
 };
 
@@ -143,8 +144,9 @@ struct VecArgs {
 template <bool ROWS>
 __device__ __forceinline__ void place(const VecArgs& a, int64_t k, uint32_t& row, int64_t& col) {
   if constexpr (ROWS) {
-    row = div32((uint32_t)k, a.cpr);
-    col = (int64_t)(((uint32_t)k - row * a.cpr.d) * 8);
+    const RowChunk c = row_chunk((uint32_t)k, a.cpr);
+    row = c.row;
+    col = c.col;
   } else {
     row = 0;
     col = k * 8;
@@ -280,7 +282,7 @@ int launch_pointwise(const char* who, int op, const void* const* in, const int64
   for (int i = 0; i < nin; ++i) flat = flat && (M == 1 || in_rs[i] == N);
   for (int i = 0; i < nout; ++i) flat = flat && (M == 1 || out_rs[i] == N);
   const int64_t n = flat ? M * N : N, rows = flat ? 1 : M, cpr = ceil_div(n, 8);
-  if (n >= 8 && (flat || cpr <= 0x7fff0000LL / rows)) {
+  if (n >= 8 && (flat || cpr <= kMaxRowChunks / rows)) {
     VecArgs a{};
     for (int i = 0; i < nin; ++i) {
       a.in[i] = static_cast<const uint16_t*>(in[i]);
