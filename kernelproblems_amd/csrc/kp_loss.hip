@@ -64,7 +64,11 @@ struct FwdArgs {
 __device__ __forceinline__ void online8(float& R, float& s, const float* v) {
   const float cm = fmaxf(fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])), fmaxf(fmaxf(v[4], v[5]), fmaxf(v[6], v[7])));
   const float rn = fmaxf(R, cm * kLog2e);  // rounding to fp32 is monotone: max commutes with it
-  if (rn == -INFINITY) return;             // nothing but -inf so far: (R, s) stays (-inf, 0)
+  if (rn == -INFINITY) {                   // nothing but -inf so far: (R, s) stays (-inf, 0), (-inf, NaN) if NaN among it
+    const float t = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+    if (t != t) s = t;
+    return;
+  }
   s *= (R == rn) ? 1.0f : __builtin_amdgcn_exp2f(R - rn);
   float c = 0.0f, d = 0.0f;
 #pragma unroll
@@ -76,10 +80,14 @@ __device__ __forceinline__ void online8(float& R, float& s, const float* v) {
   R = rn;
 }
 
-// (R1, s1) + (R2, s2) of two lanes' states.
+// (R1, s1) + (R2, s2) of two lanes' states; a NaN in s or R of either one is one in both lanes' sums.
 __device__ __forceinline__ void combine(float& R, float& s, float R2, float s2) {
   const float rn = fmaxf(R, R2);
-  if (rn == -INFINITY) return;
+  if (rn == -INFINITY) {  // 0 + 0, or NaN
+    R = rn;
+    s += s2;
+    return;
+  }
   const float a = (R == rn) ? s : s * __builtin_amdgcn_exp2f(R - rn);
   const float b = (R2 == rn) ? s2 : s2 * __builtin_amdgcn_exp2f(R2 - rn);
   R = rn;
@@ -437,7 +445,8 @@ __device__ __forceinline__ void fb_row_loss(const FbArgs& a, int64_t row, const 
 // x L - R (small for the large p), and k = g / s carries fp32 relative error.
 // The target's entry is (p - 1) g with p = exp / s divided out first: p near 1
 // (a confident row) has fp32 relative error, and p = 1 gives exactly 0.  A row
-// without a target has k = 0.
+// without a target has k = 0 / s: 0, or NaN in every column where s is 0 or
+// NaN (a row with NaN or +inf, or of -inf alone), as eager's 0 - p * 0.
 __device__ __forceinline__ float fb_exp(float x, float R) {
   return __builtin_amdgcn_exp2f(__builtin_fmaf(x, kLog2e, -R));
 }
@@ -607,7 +616,7 @@ __global__ __launch_bounds__(NT < kThreads ? kThreads : NT, KC > 8 ? 4 : 1) void
     const float xt = bf_to_f(xtb);
     row_combine<NT>(R, s, red[parity]);
     if (a.row_loss != nullptr && tid == 0) fb_row_loss(a, row, rt, R, s, xt);
-    const float kf = rt.valid ? a.g / s : 0.0f;
+    const float kf = (rt.valid ? a.g : 0.0f) / s;
     const float kl = Rl == R ? kf : kf * __builtin_amdgcn_exp2f(Rl - R);  // for the kept exponentials, against Rl
     keep_packed<KC - KE>(v + KE);
     asm volatile("" : "+v"(tid));  // the store offsets are recomputed here, not kept from the loads
@@ -670,7 +679,7 @@ __global__ __launch_bounds__(kThreads) void xent_fwd_bwd_scalar(FbArgs a) {
   asm volatile("" ::"v"(xt));  // x_t has arrived before the barrier: other waves may overwrite it after
   row_combine<kThreads>(R, s, red);
   if (a.row_loss != nullptr && threadIdx.x == 0) fb_row_loss(a, row, rt, R, s, xt);
-  const float kf = rt.valid ? a.g / s : 0.0f;
+  const float kf = (rt.valid ? a.g : 0.0f) / s;
   for (int64_t j = threadIdx.x; j < a.V; j += kThreads) {
     const float xj = bf_to_f(x[j]);
     o[j] = f_to_bf(j == rt.t ? fb_target_grad(xj, R, s, a.g) : fb_exp(xj, R) * kf);
