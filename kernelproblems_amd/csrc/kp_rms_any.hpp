@@ -81,9 +81,14 @@ __device__ __forceinline__ void any_weight(u32x4 (&wv)[VPL], const uint16_t* w, 
 // flight before the first sum (short rows would otherwise have one load per
 // lane in flight).  The weight is requested after the rows: both are in
 // flight together, and a block's few rows do not repay waiting for it first.
-template <int LPR, int VPL, int WPR, int NX, int U>
+// GATHER: term 0's row is the one that the row's id names (see RmsFwdArgs; one
+// wave-uniform id per wave), read with cacheable loads and summed in the same
+// order, so that a gathered row and the same row given directly agree bit for
+// bit.
+template <int LPR, int VPL, int WPR, int NX, int U, bool GATHER = false>
 __global__ __launch_bounds__(kThreads) void rms_fwd_any(RmsFwdArgs a) {
   static_assert(LPR == 64 || (WPR == 1 && VPL == 1), "");
+  static_assert(!GATHER || (LPR == 64 && NX == 1 && U == 1), "");
   constexpr int RW = 64 / LPR;  // rows per wave
   __shared__ float red[U][4];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -94,14 +99,21 @@ __global__ __launch_bounds__(kThreads) void rms_fwd_any(RmsFwdArgs a) {
   const int64_t row0 = ((int64_t)blockIdx.x * (4 / WPR) + rloc) * (U * RW) + rsub;
 
   u32x4 raw[U][NX][VPL];
+  bool id_ok = true;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const int64_t row = clamp_row(row0 + u * RW, a.M);
+    int64_t row = clamp_row(row0 + u * RW, a.M);
+    if constexpr (GATHER) {
+      const int64_t id = a.idx_bytes == 8 ? static_cast<const int64_t*>(a.idx)[row]
+                                          : (int64_t) static_cast<const int32_t*>(a.idx)[row];
+      id_ok = id >= 0 && id < a.idx_rows;
+      row = id_ok ? id : 0;
+    }
 #pragma unroll
     for (int t = 0; t < NX; ++t) {
       const uint16_t* p = a.x[t] + row * a.xs[t];
 #pragma unroll
-      for (int i = 0; i < VPL; ++i) raw[u][t][i] = ld16u_stream(p + cols.start[i]);
+      for (int i = 0; i < VPL; ++i) raw[u][t][i] = GATHER ? ld16u(p + cols.start[i]) : ld16u_stream(p + cols.start[i]);
     }
   }
   u32x4 wv[VPL];
@@ -118,6 +130,7 @@ __global__ __launch_bounds__(kThreads) void rms_fwd_any(RmsFwdArgs a) {
       u32x4 s = raw[u][0][i];
 #pragma unroll
       for (int t = 1; t < NX; ++t) s = add_bf8(s, raw[u][t][i]);
+      if (GATHER && !id_ok) s = u32x4{0u, 0u, 0u, 0u};
       hv[u][i] = s;
       float f[8];
       unpack8(s, f);
@@ -149,7 +162,7 @@ __global__ __launch_bounds__(kThreads) void rms_fwd_any(RmsFwdArgs a) {
     if (row >= a.M) continue;
     const float r = 1.0f / sqrtf(ss[u] / (float)a.N + a.eps);
     uint16_t* yrow = a.y + row * a.ys;
-    uint16_t* hrow = NX > 1 && a.h != nullptr ? a.h + row * a.hs : nullptr;
+    uint16_t* hrow = (NX > 1 || GATHER) && a.h != nullptr ? a.h + row * a.hs : nullptr;
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
       float h[8], w[8], o[8];
@@ -163,6 +176,7 @@ __global__ __launch_bounds__(kThreads) void rms_fwd_any(RmsFwdArgs a) {
       }
     }
     if (a.rstd != nullptr && part == 0 && sub == 0) a.rstd[row] = r;
+    if (GATHER && !id_ok && part == 0 && sub == 0 && a.err) *a.err = 1;
   }
 }
 
@@ -437,6 +451,7 @@ __global__ __launch_bounds__(kAnyWaves * 64) void rms_bwd_any(RmsBwdArgs a) {
 // Kernels for a shape and term counts, or nullptr (kp_rms_fwd_any.hip,
 // kp_rms_bwd_any_1.hip, kp_rms_bwd_any_2.hip).
 FwdKernel fwd_any_kernel(const AnyShape& s, int nx);
+FwdKernel fwd_any_gather_kernel(const AnyShape& s);  // four waves per row, at most 8192 columns
 FwdKernel fwd_any_loop_kernel(const AnyShape& s, int nx);
 BwdKernel bwd_any_kernel_short(const AnyShape& s, int nx, int ndy, bool res);
 BwdKernel bwd_any_kernel_wide(const AnyShape& s, int nx, int ndy, bool res);

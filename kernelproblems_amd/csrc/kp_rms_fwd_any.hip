@@ -52,6 +52,15 @@ FwdKernel fwd_any_kernel(const AnyShape& s, int nx) {
   return nullptr;
 }
 
+FwdKernel fwd_any_gather_kernel(const AnyShape& s) {
+  switch (s.lpr * 100 + s.vpl * 10 + s.wpr) {
+    case 6424: return rms_fwd_any<64, 2, 4, 1, 1, true>;
+    case 6434: return rms_fwd_any<64, 3, 4, 1, 1, true>;
+    case 6444: return rms_fwd_any<64, 4, 4, 1, 1, true>;
+  }
+  return nullptr;
+}
+
 FwdKernel fwd_any_loop_kernel(const AnyShape& s, int nx) {
   switch (s.vpl * 10 + s.wpr) {
     case 31: return loop_for<3, 1>(nx);

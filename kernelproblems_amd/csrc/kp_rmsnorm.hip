@@ -245,6 +245,14 @@ bool pick_fwd(int64_t M, int64_t N, int* vpl, int* wpr) {
   return true;
 }
 
+// A few wide rows: four waves per row from the kernels for any width, a block
+// per row, finish sooner than a row's one or two waves, and without the large
+// grid's starting pause (two terms, 16 rows: 4096 columns 4.0 -> 2.7 us, 2560
+// 3.1 -> 2.6, 8192 3.5 -> 3.1; 256 rows of 4096 5.1 -> 3.7, 1024 rows 7.1
+// both).  The forward and the gathered forward share the rule, so that a
+// gathered row has the bits of the same row given directly.
+bool few_wide_rows(int64_t M, int64_t N) { return N > 2048 && M <= cu_count(); }
+
 // Backward row shape: N = 8192 runs 8 waves per row with 2 chunks per lane in
 // 8-wave blocks (one row per block step; measured on MI355X at [16384, 8192]
 // with two x terms: 171.5 us against 175.5 us for 4 waves x 4 chunks in
@@ -575,12 +583,7 @@ int kp_rmsnorm_fwd_bf16(const void* const* x_terms, const int64_t* x_strides, in
   bool vec = pick_fwd(M, N, &vpl, &wpr) && rows_vec_ok(x_terms, x_strides, n_x) && aligned16(y) && (y_stride & 7) == 0;
   if (vec && h_out) vec = aligned16(h_out) && (h_stride & 7) == 0;
   if (vec && weight) vec = aligned16(weight) && (w_seg_len & 7) == 0 && (w_seg_stride & 7) == 0;
-  // A few wide rows: four waves per row from the kernels for any width, a block
-  // per row, finish sooner than a row's one or two waves, and without the
-  // large grid's starting pause (two terms, 16 rows: 4096 columns 4.0 -> 2.7
-  // us, 2560 3.1 -> 2.6, 8192 3.5 -> 3.1; 256 rows of 4096 5.1 -> 3.7, 1024
-  // rows 7.1 both).
-  vec = vec && !(M <= cu_count() && N > 2048);
+  vec = vec && !few_wide_rows(M, N);
   const FwdKernel fk = vec ? fwd_kernel(vpl, wpr, n_x) : nullptr;
   vec = vec && fk != nullptr;
   hipStream_t s = as_stream(stream);
@@ -666,9 +669,9 @@ int kp_embedding_rmsnorm_fwd_bf16(const void* table, int64_t V, int64_t table_ro
   a.eps = eps;
 
   int vpl = 0, wpr = 0;
-  // one wave per row whatever T: the gather's row-per-block form measured
-  // 39.3 against 34.2 us at C3 (cache-served table rows favour the
-  // persistent pipelined grid)
+  // one wave per row beyond a few (few_wide_rows): the gather's row-per-block
+  // form measured 39.3 against 34.2 us at C3 (cache-served table rows favour
+  // the persistent pipelined grid)
   bool vec = pick_vec(N, true, &vpl, &wpr) && aligned16(table) && (table_row_stride & 7) == 0 && aligned16(y) &&
              (y_stride & 7) == 0;
   if (vec && h_out) vec = aligned16(h_out) && (h_stride & 7) == 0;
@@ -676,6 +679,15 @@ int kp_embedding_rmsnorm_fwd_bf16(const void* table, int64_t V, int64_t table_ro
   const FwdKernel fk = vec ? fwd_gather_kernel(vpl, wpr) : nullptr;
   if (fk == nullptr)
     return fail(KP_EUNSUPPORTED, "%s: row shape / alignment without a fused kernel (N=%lld)", who, (long long)N);
+  AnyShape as{};
+  if (few_wide_rows(T, N) && any_fwd_shape(T, N, cu_count(), &as)) {
+    if (const FwdKernel ak = fwd_any_gather_kernel(as)) {
+      void* args[] = {&a};
+      launch_dominant_raw(reinterpret_cast<const void*>(ak), dim3((unsigned)T), dim3(kThreads), args, 0,
+                          as_stream(stream));
+      return check_launch(who);
+    }
+  }
   const int rb = 4 / wpr;
   const int64_t groups = ceil_div(T, rb);
   // one block per row for rows of 4 waves, as in kp_rmsnorm_fwd_bf16
