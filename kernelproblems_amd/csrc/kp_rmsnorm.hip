@@ -327,11 +327,12 @@ size_t bwd_workspace_size(int64_t M, int64_t N) {
   const int64_t rows = M < blocks ? M : blocks;
   return (size_t)(rows * ceil_div(N, kPartChunk) * kPartChunk * (int64_t)sizeof(float));
 }
-// The fused forward + backward's size has room for an fp32 rstd per row after
-// the partial rows, as callers have allocated it.
+size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
+// The fused forward + backward also keeps room for an fp32 rstd per row after
+// the partial rows (used only by its two-launch fallback).
 size_t fwd_bwd_workspace_size(int64_t M, int64_t N) {
   if (M <= 0 || N <= 0) return 16;
-  return ((bwd_workspace_size(M, N) + 255) & ~(size_t)255) + (size_t)M * sizeof(float);
+  return align256(bwd_workspace_size(M, N)) + (size_t)M * sizeof(float);
 }
 
 // Launch plan of a backward row pass: the kernel and its block count (each
@@ -384,13 +385,101 @@ size_t partial_bytes(const BwdPlan& p, int64_t N) {
   return (size_t)p.blocks * (size_t)(ceil_div(N, kPartChunk) * kPartChunk) * sizeof(float);
 }
 
+// The RMSNorm forward.  few_rows false: without the layout of a few wide rows.
+int rms_fwd_impl(const char* who, const void* const* x_terms, const int64_t* x_strides, int n_x, const void* weight,
+                 int64_t w_seg_len, int64_t w_seg_stride, void* h_out, int64_t h_stride, void* y, int64_t y_stride,
+                 float* rstd, int64_t M, int64_t N, float eps, bool few_rows, void* stream) {
+  int st = check_terms(who, "x", x_terms, x_strides, n_x, M);
+  if (st != KP_OK) return st;
+  if (M < 0 || N <= 0) return fail(KP_EINVAL, "%s: need M >= 0 and N > 0 (M=%lld N=%lld)", who, (long long)M, (long long)N);
+  if ((y == nullptr && M > 0) || y_stride < 0) return fail(KP_EINVAL, "%s: y is NULL or has a negative stride", who);
+  if (weight != nullptr && (w_seg_len <= 0 || w_seg_stride < 0))
+    return fail(KP_EINVAL, "%s: weight segment length must be > 0", who);
+  if (M == 0) return KP_OK;
+
+  RmsFwdArgs a{};
+  for (int i = 0; i < n_x; ++i) {
+    a.x[i] = static_cast<const uint16_t*>(x_terms[i]);
+    a.xs[i] = x_strides[i];
+  }
+  a.n_x = n_x;
+  a.w = static_cast<const uint16_t*>(weight);
+  a.w_seg_len = weight ? w_seg_len : N;
+  a.w_seg_stride = weight ? w_seg_stride : N;
+  a.h = static_cast<uint16_t*>(h_out);
+  a.hs = h_stride;
+  a.y = static_cast<uint16_t*>(y);
+  a.ys = y_stride;
+  a.rstd = rstd;
+  a.M = M;
+  a.N = N;
+  a.eps = eps;
+
+  int vpl = 0, wpr = 0;
+  bool vec = pick_fwd(M, N, &vpl, &wpr) && rows_vec_ok(x_terms, x_strides, n_x) && aligned16(y) && (y_stride & 7) == 0;
+  if (vec && h_out) vec = aligned16(h_out) && (h_stride & 7) == 0;
+  if (vec && weight) vec = aligned16(weight) && (w_seg_len & 7) == 0 && (w_seg_stride & 7) == 0;
+  vec = vec && !(few_rows && few_wide_rows(M, N));
+  const FwdKernel fk = vec ? fwd_kernel(vpl, wpr, n_x) : nullptr;
+  vec = vec && fk != nullptr;
+  hipStream_t s = as_stream(stream);
+  if (vec) {
+    const int rb = 4 / wpr;
+    const int64_t groups = ceil_div(M, rb);
+    // Rows of 4 waves (one row per block): one block per row, no persistent
+    // walk -- measured on MI355X at [16384, 8192] with two x terms: 170.5 us
+    // against 185 us for 2 pipelined blocks per CU.  Shorter rows (1 or 2
+    // waves) keep the pipelined grid ([4096, 4096]: 12.5 us against 13.8 us
+    // for one block per 4 rows).
+    const int64_t cap = wpr == 4 ? groups : (int64_t)cu_count() * fwd_bpc((int64_t)n_x * vpl * 1024);
+    if (groups > INT32_MAX) return fail(KP_EUNSUPPORTED, "%s: too many rows for one launch", who);
+    const int grid = (int)(groups < cap ? groups : cap);
+    void* args[] = {&a};
+    launch_dominant_raw(reinterpret_cast<const void*>(fk), dim3(grid), dim3(kThreads), args, 0, s);
+    return check_launch(who);
+  }
+  // Any width and alignment.  Rows of middling width, more of them than CUs,
+  // run the persistent loop (us, one-shot / loop: [3001, 2880] two terms 14.0 /
+  // 12.3, [4096, 4095] 15.8 / 13.8, [16384, 2881] two terms 79.8 / 72.5); few
+  // or short rows are as fast or faster with a block each ([2048, 1001] two
+  // terms 4.9 / 5.2), wider ones too ([8192, 5121] two terms 72.0 / 74.9), and
+  // so are rows on 16-byte addresses once the call's traffic is beyond the
+  // Infinity Cache ([8192, 5120] two terms 56.0 / 58.9).
+  AnyShape as{}, ls{};
+  const FwdKernel ak = any_fwd_shape(M * n_x, N, cu_count(), &as) ? fwd_any_kernel(as, n_x) : nullptr;
+  const bool streamed = (N & 7) == 0 && rows_vec_ok(x_terms, x_strides, n_x) &&
+                        M * N * 2 * (n_x + (n_x > 1 && h_out != nullptr ? 2 : 1)) > ((int64_t)160 << 20);
+  const FwdKernel lk = M > cu_count() && !streamed && any_loop_shape(N, &ls) ? fwd_any_loop_kernel(ls, n_x) : nullptr;
+  if (lk != nullptr) {
+    const int64_t lgroups = ceil_div(M, 4 / ls.wpr), cap = (int64_t)cu_count() * fwd_bpc((int64_t)n_x * ls.vpl * 1024);
+    void* args[] = {&a};
+    launch_dominant_raw(reinterpret_cast<const void*>(lk), dim3((unsigned)(lgroups < cap ? lgroups : cap)),
+                        dim3(kThreads), args, 0, s);
+    return check_launch(who);
+  }
+  const int64_t groups = ak != nullptr ? ceil_div(M, (int64_t)(4 / as.wpr) * (64 / as.lpr) * as.u) : 0;
+  if (ak != nullptr && groups <= max_blocks(kThreads)) {
+    void* args[] = {&a};
+    launch_dominant_raw(reinterpret_cast<const void*>(ak), dim3((unsigned)groups), dim3(kThreads), args, 0, s);
+  } else {
+    const int64_t cap = (int64_t)cu_count() * 8;
+    const int grid = (int)(M < cap ? M : cap);
+    KP_LAUNCH_DOMINANT(rms_fwd_generic, dim3(grid), dim3(kThreads), 0, s, a);
+  }
+  return check_launch(who);
+}
+
 // The RMSNorm backward (fo == nullptr) and the fused forward + backward
 // (fo != nullptr: rstd is recomputed and y / h / rstd are written by the same
 // row pass).  Shapes or term combinations without a fused kernel run the
-// forward kernel and then the backward, which recomputes rstd: the rows'
-// layouts may differ, and so the last bit of a sum, and dx and dw are to be
-// those of the backward called without rstd.  The workspace must hold the partial rows the launch plan writes (the *_size
-// functions return an upper bound of that).
+// forward kernel and then the backward with the rstd it wrote, so that both
+// halves use one (their row layouts may differ, and so the last bit of a sum):
+// in rstd_out or, when the caller wants none, in the workspace past the
+// partial rows, where the *_size function has room for it (a smaller
+// workspace: the backward recomputes it).  The forward keeps the backward's
+// layout where both have N = 512 * k kernels of it.  The workspace must hold
+// the partial rows the launch plan writes (the *_size functions return an
+// upper bound of that).
 int rms_bwd_impl(const char* who, const void* const* dy_terms, const int64_t* dy_strides, int n_dy,
                  const void* const* x_terms, const int64_t* x_strides, int n_x, const float* rstd, const void* weight,
                  int64_t w_seg_len, int64_t w_seg_stride, const void* dx_residual, int64_t dxr_stride, void* dx,
@@ -449,9 +538,14 @@ int rms_bwd_impl(const char* who, const void* const* dy_terms, const int64_t* dy
 
   if (M > 0) {
     if (two_launch) {
-      st = kp_rmsnorm_fwd_bf16(x_terms, x_strides, n_x, weight, w_seg_len, w_seg_stride, n_x > 1 ? fo->h : nullptr,
-                               fo->hs, fo->y, fo->ys, fo->rstd, M, N, eps, stream);
+      const size_t at = align256(need);
+      float* r = fo->rstd;
+      if (r == nullptr && workspace != nullptr && aligned16(workspace) && workspace_bytes >= at + (size_t)M * sizeof(float))
+        r = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + at);
+      st = rms_fwd_impl(who, x_terms, x_strides, n_x, weight, w_seg_len, w_seg_stride, n_x > 1 ? fo->h : nullptr,
+                        fo->hs, fo->y, fo->ys, r, M, N, eps, plan.vec == nullptr, stream);
       if (st != KP_OK) return st;
+      a.rstd = r;
     } else if (fo != nullptr) {
       a.y = fo->y;
       a.ys = fo->ys;
@@ -552,85 +646,8 @@ extern "C" {
 int kp_rmsnorm_fwd_bf16(const void* const* x_terms, const int64_t* x_strides, int n_x, const void* weight,
                         int64_t w_seg_len, int64_t w_seg_stride, void* h_out, int64_t h_stride, void* y,
                         int64_t y_stride, float* rstd, int64_t M, int64_t N, float eps, void* stream) {
-  static const char* who = "kp_rmsnorm_fwd_bf16";
-  int st = check_terms(who, "x", x_terms, x_strides, n_x, M);
-  if (st != KP_OK) return st;
-  if (M < 0 || N <= 0) return fail(KP_EINVAL, "%s: need M >= 0 and N > 0 (M=%lld N=%lld)", who, (long long)M, (long long)N);
-  if ((y == nullptr && M > 0) || y_stride < 0) return fail(KP_EINVAL, "%s: y is NULL or has a negative stride", who);
-  if (weight != nullptr && (w_seg_len <= 0 || w_seg_stride < 0))
-    return fail(KP_EINVAL, "%s: weight segment length must be > 0", who);
-  if (M == 0) return KP_OK;
-
-  RmsFwdArgs a{};
-  for (int i = 0; i < n_x; ++i) {
-    a.x[i] = static_cast<const uint16_t*>(x_terms[i]);
-    a.xs[i] = x_strides[i];
-  }
-  a.n_x = n_x;
-  a.w = static_cast<const uint16_t*>(weight);
-  a.w_seg_len = weight ? w_seg_len : N;
-  a.w_seg_stride = weight ? w_seg_stride : N;
-  a.h = static_cast<uint16_t*>(h_out);
-  a.hs = h_stride;
-  a.y = static_cast<uint16_t*>(y);
-  a.ys = y_stride;
-  a.rstd = rstd;
-  a.M = M;
-  a.N = N;
-  a.eps = eps;
-
-  int vpl = 0, wpr = 0;
-  bool vec = pick_fwd(M, N, &vpl, &wpr) && rows_vec_ok(x_terms, x_strides, n_x) && aligned16(y) && (y_stride & 7) == 0;
-  if (vec && h_out) vec = aligned16(h_out) && (h_stride & 7) == 0;
-  if (vec && weight) vec = aligned16(weight) && (w_seg_len & 7) == 0 && (w_seg_stride & 7) == 0;
-  vec = vec && !few_wide_rows(M, N);
-  const FwdKernel fk = vec ? fwd_kernel(vpl, wpr, n_x) : nullptr;
-  vec = vec && fk != nullptr;
-  hipStream_t s = as_stream(stream);
-  if (vec) {
-    const int rb = 4 / wpr;
-    const int64_t groups = ceil_div(M, rb);
-    // Rows of 4 waves (one row per block): one block per row, no persistent
-    // walk -- measured on MI355X at [16384, 8192] with two x terms: 170.5 us
-    // against 185 us for 2 pipelined blocks per CU.  Shorter rows (1 or 2
-    // waves) keep the pipelined grid ([4096, 4096]: 12.5 us against 13.8 us
-    // for one block per 4 rows).
-    const int64_t cap = wpr == 4 ? groups : (int64_t)cu_count() * fwd_bpc((int64_t)n_x * vpl * 1024);
-    if (groups > INT32_MAX) return fail(KP_EUNSUPPORTED, "%s: too many rows for one launch", who);
-    const int grid = (int)(groups < cap ? groups : cap);
-    void* args[] = {&a};
-    launch_dominant_raw(reinterpret_cast<const void*>(fk), dim3(grid), dim3(kThreads), args, 0, s);
-    return check_launch(who);
-  }
-  // Any width and alignment.  Rows of middling width, more of them than CUs,
-  // run the persistent loop (us, one-shot / loop: [3001, 2880] two terms 14.0 /
-  // 12.3, [4096, 4095] 15.8 / 13.8, [16384, 2881] two terms 79.8 / 72.5); few
-  // or short rows are as fast or faster with a block each ([2048, 1001] two
-  // terms 4.9 / 5.2), wider ones too ([8192, 5121] two terms 72.0 / 74.9), and
-  // so are rows on 16-byte addresses once the call's traffic is beyond the
-  // Infinity Cache ([8192, 5120] two terms 56.0 / 58.9).
-  AnyShape as{}, ls{};
-  const FwdKernel ak = any_fwd_shape(M * n_x, N, cu_count(), &as) ? fwd_any_kernel(as, n_x) : nullptr;
-  const bool streamed = (N & 7) == 0 && rows_vec_ok(x_terms, x_strides, n_x) &&
-                        M * N * 2 * (n_x + (n_x > 1 && h_out != nullptr ? 2 : 1)) > ((int64_t)160 << 20);
-  const FwdKernel lk = M > cu_count() && !streamed && any_loop_shape(N, &ls) ? fwd_any_loop_kernel(ls, n_x) : nullptr;
-  if (lk != nullptr) {
-    const int64_t lgroups = ceil_div(M, 4 / ls.wpr), cap = (int64_t)cu_count() * fwd_bpc((int64_t)n_x * ls.vpl * 1024);
-    void* args[] = {&a};
-    launch_dominant_raw(reinterpret_cast<const void*>(lk), dim3((unsigned)(lgroups < cap ? lgroups : cap)),
-                        dim3(kThreads), args, 0, s);
-    return check_launch(who);
-  }
-  const int64_t groups = ak != nullptr ? ceil_div(M, (int64_t)(4 / as.wpr) * (64 / as.lpr) * as.u) : 0;
-  if (ak != nullptr && groups <= max_blocks(kThreads)) {
-    void* args[] = {&a};
-    launch_dominant_raw(reinterpret_cast<const void*>(ak), dim3((unsigned)groups), dim3(kThreads), args, 0, s);
-  } else {
-    const int64_t cap = (int64_t)cu_count() * 8;
-    const int grid = (int)(M < cap ? M : cap);
-    KP_LAUNCH_DOMINANT(rms_fwd_generic, dim3(grid), dim3(kThreads), 0, s, a);
-  }
-  return check_launch(who);
+  return rms_fwd_impl("kp_rmsnorm_fwd_bf16", x_terms, x_strides, n_x, weight, w_seg_len, w_seg_stride, h_out, h_stride,
+                      y, y_stride, rstd, M, N, eps, true, stream);
 }
 
 int kp_embedding_rmsnorm_fwd_bf16(const void* table, int64_t V, int64_t table_row_stride, const void* indices,
