@@ -710,6 +710,26 @@ FbPlan fb_plan(int64_t V) {
 
 bool valid_target_bytes(int b) { return b == 4 || b == 8; }
 
+// Threads per row of the forward: a wave while there are rows enough to fill
+// the chip, else a block (a wave streams a row at a few GB/s by itself).  A
+// block's start and reduction weigh the more the shorter the row, a second
+// step of 256 threads (16384 elements each) that is less than half full idles,
+// and rows at any address leave fewer lines in flight, so the line lies at 2,
+// 3, 4 or 6 rows per CU.  Measured on MI355X (256 CUs), per call of both
+// launches, a wave / 256 threads (us): V = 12288 512 rows 12.0 / 10.7, 768
+// 12.2 / 12.3; 16384 1280 rows 16.2 / 15.3, 1600 16.6 / 17.4; 18432 768 rows
+// 14.6 / 13.6, 1024 15.2 / 15.8, 1815 18.1 / 22.1; 24576 1536 20.4 / 18.5; 32768
+// 1536 rows 25.8 / 22.2; 50256 1536 rows 34.4 / 33.4, 1600 34.7 / 36.9; 90880
+// 1815 rows 57.3 / 63.2; rows not 16-byte aligned: 24577 1024 rows 19.5 /
+// 18.6, 1152 21.5 / 21.9; 50257 1024 rows 31.8 / 28.7, 1408 35.3 / 38.4;
+// 1024 threads, 256 / 1024: 128256 256 rows 26.6 / 18.1, 512 30.8 / 28.0, 768
+// 37.9 / 37.7; 90880 512 rows 24.9 / 23.0; 18432 256 rows 10.5 / 11.2.
+int fwd_threads(int64_t M, int64_t V, bool aligned, int cus) {
+  const int64_t per_cu = V < 16384 ? 2 : V > 16384 && V < 24576 ? 3 : aligned ? 6 : 4;
+  if (V < 8192 || M > per_cu * cus) return 64;
+  return M < (int64_t)2 * cus && V >= 32768 ? 1024 : 256;
+}
+
 }  // namespace
 }  // namespace kp
 
@@ -751,9 +771,8 @@ int kp_cross_entropy_fwd_bf16(const void* logits, int64_t row_stride, int64_t M,
   a.lse_out = row_lse;
   a.err = error_flag;
   if (M > 0) {
-    // Threads per row: a wave while there are rows enough to fill the chip,
-    // then a block (a wave streams a row at a few GB/s by itself).
-    const int nt = V < 8 ? 0 : M >= 2048 || V < 8192 ? 64 : M >= 512 || V < 32768 ? 256 : 1024;
+    const bool aligned = aligned16(logits) && (M == 1 || row_stride % 8 == 0);
+    const int nt = V < 8 ? 0 : fwd_threads(M, V, aligned, cu_count());
     const void* fk = nt == 0     ? reinterpret_cast<const void*>(xent_fwd_scalar)
                      : nt == 64  ? reinterpret_cast<const void*>(xent_fwd_vec<64>)
                      : nt == 256 ? reinterpret_cast<const void*>(xent_fwd_vec<256>)
