@@ -250,43 +250,65 @@ __global__ __launch_bounds__(kThreads) void xent_fwd_scalar(FwdArgs a) {
   if (lane == 0) finish_row(a, row, rt, R, s);
 }
 
-// One block: loss = scale * sum(row_loss), total_weight = sum(row_valid), in a
-// fixed order: thread t sums rows t, t + 1024, ... in fp64 (four of them
-// requested together), lanes fold by shuffles, then the first wave folds the
-// 16 wave sums (one barrier; a tree through LDS with a barrier per level
-// made this launch 4.2 us).
-constexpr int kFinThreads = 1024;
-__device__ __forceinline__ double wave_sum_f64(double v) {
-#pragma unroll
-  for (int m = 1; m < kWave; m <<= 1) v += __shfl_xor(v, m, kWave);
+// Sum of one double over the 64 lanes, the same tree and order as wave_sum.
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xF, 0xF, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xF, 0xF, true);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ double readlane_d(double v, int lane) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), lane);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ double row16_sum_d(double v) {
+  v += dpp_d<0xB1>(v);
+  v += dpp_d<0x4E>(v);
+  v += dpp_d<0x141>(v);
+  v += dpp_d<0x140>(v);
   return v;
 }
+__device__ __forceinline__ double wave_sum_d(double v) {
+  v = row16_sum_d(v);
+  return (readlane_d(v, 0) + readlane_d(v, 16)) + (readlane_d(v, 32) + readlane_d(v, 48));
+}
+
+// One block: loss = scale * sum(row_loss), total_weight = sum(row_valid), in a
+// fixed order: thread t sums rows t, t + 1024, ... in fp64, four of them
+// requested together (past the last row: the last one again, not added); lanes
+// fold by DPP and readlane, then the 16 lanes of a DPP row fold the 16 wave
+// sums (one barrier).  A chain of latencies, us at 64 / 2795 / 4096 / 16384 rows:
+// 1.5 / 2.0 / 2.1 / 3.9; folding by __shfl_xor (an LDS round trip a step) and
+// one load at a time below 4096 rows 2.5 / 3.2 / 3.8 / 4.8, a tree through LDS
+// with a barrier per level 2.1 / 2.9 / 3.2 / 6.8.
+constexpr int kFinThreads = 1024;
 __global__ __launch_bounds__(kFinThreads) void xent_fwd_finish(const double* row_loss, const int32_t* row_valid,
                                                                 int64_t M, double scale, float* loss, float* total_weight) {
   constexpr int kW = kFinThreads / kWave;
+  static_assert(kW == 16, "");
   __shared__ double ls[kW], cs[kW];
   double acc = 0.0, cnt = 0.0;  // counts below 2^53 are exact in any order
-  int64_t i = threadIdx.x;
-  for (; i + 3 * kFinThreads < M; i += 4 * kFinThreads) {
+  for (int64_t i = threadIdx.x; i < M; i += 4 * kFinThreads) {
     double l[4];
     int32_t c[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      l[k] = row_loss[i + k * kFinThreads];
-      c[k] = row_valid[i + k * kFinThreads];
+      const int64_t r = i + k * kFinThreads < M ? i + k * kFinThreads : M - 1;
+      l[k] = row_loss[r];
+      c[k] = row_valid[r];
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      acc += l[k];
-      cnt += (double)c[k];
+      const bool in = i + k * kFinThreads < M;
+      acc = in ? acc + l[k] : acc;
+      cnt += in ? (double)c[k] : 0.0;
     }
   }
-  for (; i < M; i += kFinThreads) {
-    acc += row_loss[i];
-    cnt += (double)row_valid[i];
-  }
-  acc = wave_sum_f64(acc);
-  cnt = wave_sum_f64(cnt);
+  acc = wave_sum_d(acc);
+  cnt = wave_sum_d(cnt);
   const int lane = threadIdx.x & (kWave - 1);
   if (lane == 0) {
     ls[threadIdx.x >> 6] = acc;
@@ -294,8 +316,8 @@ __global__ __launch_bounds__(kFinThreads) void xent_fwd_finish(const double* row
   }
   __syncthreads();
   if (threadIdx.x >= kWave) return;
-  acc = wave_sum_f64(lane < kW ? ls[lane] : 0.0);
-  cnt = wave_sum_f64(lane < kW ? cs[lane] : 0.0);
+  acc = row16_sum_d(ls[lane & (kW - 1)]);
+  cnt = row16_sum_d(cs[lane & (kW - 1)]);
   if (lane == 0) {
     loss[0] = (float)(acc * scale);
     total_weight[0] = (float)cnt;
