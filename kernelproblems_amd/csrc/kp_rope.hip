@@ -14,11 +14,11 @@
 // Work unit = one 16-byte chunk per rotation operand: rotate-half pairs chunk
 // [c*8, c*8+8) with [D/2 + c*8, ...); interleaved pairs are the 4 (2i, 2i+1)
 // pairs inside one chunk.  Arithmetic is fp32, one RNE rounding to bf16.
-#include <math.h>
 #include <stdlib.h>
 
 #include "kp_common.hpp"
 #include "kp_internal.hpp"
+#include "kp_rope_freqs.hpp"
 
 namespace kp {
 namespace {
@@ -48,11 +48,19 @@ struct RopeArgs {
   int64_t frows, frs;  // rows, row stride in complex elements
   int conj;
   int32_t* err;
-  // theta mode: inv_freq[f] = fp32(theta^(-2f/D)), evaluated once per call on
-  // the host instead of in every wave (every kernel reads it, so their angles
-  // stay identical)
-  float inv_freq[kMaxHalf];
 };
+
+// theta mode: f[i] = fp32(theta^(-2i/D)), evaluated once per call on the host
+// instead of in every wave (every kernel reads it, so their angles stay
+// identical).  A kernel's last argument, of no more entries than it needs
+// (none in table mode, 64 for D <= 128): a call of few positions is bound by
+// its host time.  16 tokens of 32 + 8 heads of 64 from theta: 5.65 us with all
+// 256 in every call's arguments and 16 + D / 32 powers, 5.45 us so.
+template <int F>
+struct InvFreq {
+  float f[F];
+};
+constexpr int inv_entries(bool table, int64_t D) { return table ? 1 : D <= 128 ? 64 : kMaxHalf; }
 
 // Output element offset o gets 8 values (16-byte bf16 / 32-byte fp32) or 1 value.
 __device__ __forceinline__ void store8p(void* out, int out_f32, int64_t o, const float* v) {
@@ -93,7 +101,7 @@ __device__ __forceinline__ void rot(float a, float b, float c, float s, float& o
 // one address space (global table or LDS slot); a runtime choice lets the
 // compiler merge both into one flat load.
 template <bool TABLE>
-__global__ __launch_bounds__(kThreads) void rope_scalar(RopeArgs a) {
+__global__ __launch_bounds__(kThreads) void rope_scalar(RopeArgs a, InvFreq<TABLE ? 1 : kMaxHalf> iv) {
   __shared__ float cs[kWavesPerBlock][2][kMaxHalf];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -102,7 +110,7 @@ __global__ __launch_bounds__(kThreads) void rope_scalar(RopeArgs a) {
   // inv_freq[f] for f = lane + 64k (theta mode), kept in registers.
   float inv[kMaxHalf / 64];
 #pragma unroll
-  for (int k = 0; k < kMaxHalf / 64; ++k) inv[k] = TABLE ? 0.f : a.inv_freq[lane + 64 * k];
+  for (int k = 0; k < kMaxHalf / 64; ++k) inv[k] = TABLE ? 0.f : iv.f[TABLE ? 0 : lane + 64 * k];
 
   const int64_t npos = a.B * a.S;
   const int64_t w0 = (int64_t)blockIdx.x * kWavesPerBlock + wave;
@@ -192,9 +200,9 @@ __global__ __launch_bounds__(kThreads) void rope_scalar(RopeArgs a) {
 // with 64-bit divisions that these widths ran before: [3, 1009, 24 + 8, 64]
 // interleaved table 8.1 -> 6.8 us, [4, 4096, 32 + 8, 64] rotate-half 38.1 ->
 // 27.0 us, [4, 4096, 16 + 4, 80] interleaved 25.8 -> 18.1 us.
-template <int PAIRING, bool TABLE, int UPL>
+template <int PAIRING, bool TABLE, int UPL, int F>
 __global__ __launch_bounds__(kThreads) void rope_wave(RopeArgs a, Div32 by_c, Div32 by_s, uint32_t step,
-                                                       uint32_t first) {
+                                                       uint32_t first, InvFreq<F> iv) {
   constexpr bool kHalf = PAIRING == KP_ROPE_HALF;
   constexpr int FPU = kHalf ? 8 : 4;  // angles per unit
   constexpr bool kStage = !TABLE || kHalf;
@@ -221,7 +229,7 @@ __global__ __launch_bounds__(kThreads) void rope_wave(RopeArgs a, Div32 by_c, Di
   int64_t p = s;
   if (a.pos) p = a.pb == 8 ? static_cast<const int64_t*>(a.pos)[b * a.psb + s * a.pss]
                            : (int64_t) static_cast<const int32_t*>(a.pos)[b * a.psb + s * a.pss];
-  const float inv0 = TABLE ? 0.f : a.inv_freq[lane];
+  const float inv0 = TABLE ? 0.f : iv.f[TABLE ? 0 : lane];
   __builtin_amdgcn_sched_barrier(0);
   bool ok = true;
   const float* frow = a.freqs;
@@ -255,7 +263,7 @@ __global__ __launch_bounds__(kThreads) void rope_wave(RopeArgs a, Div32 by_c, Di
             cn = frow[2 * f];
             sn = frow[2 * f + 1];
           } else {
-            sincosf((float)p * (f < 64 ? inv0 : a.inv_freq[f]), &sn, &cn);
+            sincosf((float)p * (F <= 64 || f < 64 ? inv0 : iv.f[f]), &sn, &cn);
           }
           cs[wave][0][f] = cn;
           cs[wave][1][f] = sgn * sn;
@@ -332,7 +340,7 @@ constexpr int kFastD = 128;
 constexpr int kFastMaxLoads = 16;
 
 template <int PAIRING, bool TABLE, int UPL>
-__device__ __forceinline__ void rope_fast_body(const RopeArgs& a) {
+__device__ __forceinline__ void rope_fast_body(const RopeArgs& a, const InvFreq<TABLE ? 1 : 64>& iv) {
   constexpr bool kHalf = PAIRING == KP_ROPE_HALF;
   constexpr int HD = kFastD / 2;
   constexpr int CPH = kHalf ? kFastD / 16 : kFastD / 8;  // units per head
@@ -385,7 +393,7 @@ __device__ __forceinline__ void rope_fast_body(const RopeArgs& a) {
     }
   } else {
     // lane f < D/2 produces angle f: fp32(fp32(p) * fp32(theta^(-2f/D)))
-    const float inv = a.inv_freq[lane];
+    const float inv = iv.f[lane];
     float sn, cn;
     sincosf((float)p * inv, &sn, &cn);
     cs[wave][0][lane] = cn;
@@ -449,8 +457,8 @@ __device__ __forceinline__ void rope_fast_body(const RopeArgs& a) {
 }
 
 template <int PAIRING, bool TABLE, int UPL>
-__global__ __launch_bounds__(kThreads) void rope_fast(RopeArgs a) {
-  rope_fast_body<PAIRING, TABLE, UPL>(a);
+__global__ __launch_bounds__(kThreads) void rope_fast(RopeArgs a, InvFreq<TABLE ? 1 : 64> iv) {
+  rope_fast_body<PAIRING, TABLE, UPL>(a, iv);
 }
 
 // ------------------------------------------------------------ tile path
@@ -748,31 +756,29 @@ bool tile_ok(const RopeArgs& a, bool table) {
   return true;
 }
 
-typedef void (*RopeKernel)(RopeArgs);
-
 template <int PAIRING, bool TABLE>
-RopeKernel fast_for_upl(int upl) {
+const void* fast_for_upl(int upl) {
   switch (upl) {
-    case 1: return rope_fast<PAIRING, TABLE, 1>;
-    case 2: return rope_fast<PAIRING, TABLE, 2>;
-    case 3: return rope_fast<PAIRING, TABLE, 3>;
-    case 4: return rope_fast<PAIRING, TABLE, 4>;
-    case 5: return rope_fast<PAIRING, TABLE, 5>;
-    case 6: return rope_fast<PAIRING, TABLE, 6>;
-    case 8: return rope_fast<PAIRING, TABLE, 8>;
+    case 1: return reinterpret_cast<const void*>(rope_fast<PAIRING, TABLE, 1>);
+    case 2: return reinterpret_cast<const void*>(rope_fast<PAIRING, TABLE, 2>);
+    case 3: return reinterpret_cast<const void*>(rope_fast<PAIRING, TABLE, 3>);
+    case 4: return reinterpret_cast<const void*>(rope_fast<PAIRING, TABLE, 4>);
+    case 5: return reinterpret_cast<const void*>(rope_fast<PAIRING, TABLE, 5>);
+    case 6: return reinterpret_cast<const void*>(rope_fast<PAIRING, TABLE, 6>);
+    case 8: return reinterpret_cast<const void*>(rope_fast<PAIRING, TABLE, 8>);
   }
   if constexpr (PAIRING == KP_ROPE_INTERLEAVED) {
     switch (upl) {
-      case 10: return rope_fast<PAIRING, TABLE, 10>;
-      case 12: return rope_fast<PAIRING, TABLE, 12>;
-      case 16: return rope_fast<PAIRING, TABLE, 16>;
+      case 10: return reinterpret_cast<const void*>(rope_fast<PAIRING, TABLE, 10>);
+      case 12: return reinterpret_cast<const void*>(rope_fast<PAIRING, TABLE, 12>);
+      case 16: return reinterpret_cast<const void*>(rope_fast<PAIRING, TABLE, 16>);
     }
   }
   return nullptr;
 }
 
 // The fast kernel for this call, or nullptr (then rope_wave runs).
-RopeKernel pick_fast(const RopeArgs& a, int pairing, bool table) {
+const void* pick_fast(const RopeArgs& a, int pairing, bool table) {
   if (a.D != kFastD) return nullptr;
   if (table && (!aligned16(a.freqs) || (a.frs & 1) != 0)) return nullptr;
   const bool half = pairing == KP_ROPE_HALF;
@@ -791,21 +797,28 @@ RopeKernel pick_fast(const RopeArgs& a, int pairing, bool table) {
   return table ? fast_for_upl<KP_ROPE_INTERLEAVED, true>((int)upl) : fast_for_upl<KP_ROPE_INTERLEAVED, false>((int)upl);
 }
 
-typedef void (*WaveKernel)(RopeArgs, Div32, Div32, uint32_t, uint32_t);
-
-template <int PAIRING, bool TABLE>
-WaveKernel wave_for_upl(int64_t upl) {
+template <int PAIRING, bool TABLE, int F>
+const void* wave_for_upl(int64_t upl) {
   switch (upl) {
-    case 1: return rope_wave<PAIRING, TABLE, 1>;
-    case 2: return rope_wave<PAIRING, TABLE, 2>;
-    case 3: return rope_wave<PAIRING, TABLE, 3>;
+    case 1: return reinterpret_cast<const void*>(rope_wave<PAIRING, TABLE, 1, F>);
+    case 2: return reinterpret_cast<const void*>(rope_wave<PAIRING, TABLE, 2, F>);
   }
-  return rope_wave<PAIRING, TABLE, 4>;
+  if constexpr (PAIRING == KP_ROPE_HALF) {
+    if (upl == 3) return reinterpret_cast<const void*>(rope_wave<PAIRING, TABLE, 3, F>);
+    return reinterpret_cast<const void*>(rope_wave<PAIRING, TABLE, 4, F>);
+  }
+  return nullptr;
+}
+template <int PAIRING>
+const void* wave_kernel(int64_t upl, int entries) {
+  return entries == 1    ? wave_for_upl<PAIRING, true, 1>(upl)
+         : entries == 64 ? wave_for_upl<PAIRING, false, 64>(upl)
+                         : wave_for_upl<PAIRING, false, kMaxHalf>(upl);
 }
 
 // The wave kernel for this call, or nullptr (D of no whole chunks, or more
 // positions or units than 32-bit indexes hold: then rope_scalar runs).
-WaveKernel pick_wave(const RopeArgs& a, int pairing, bool table, Div32* by_c, Div32* by_s, uint32_t* step) {
+const void* pick_wave(const RopeArgs& a, int pairing, bool table, Div32* by_c, Div32* by_s, uint32_t* step) {
   const bool half = pairing == KP_ROPE_HALF;
   if (a.D % (half ? 16 : 8) != 0) return nullptr;
   const int64_t cph = a.D / 8, H = a.t[0].H + (a.nt > 1 ? a.t[1].H : 0);
@@ -819,20 +832,8 @@ WaveKernel pick_wave(const RopeArgs& a, int pairing, bool table, Div32* by_c, Di
   const int64_t most = half ? 4 : 2;
   if (upl > most) upl = most;
   *step = (uint32_t)(64 * upl / cph * cph);  // whole heads (a head is at most 64 chunks)
-  if (half) return table ? wave_for_upl<KP_ROPE_HALF, true>(upl) : wave_for_upl<KP_ROPE_HALF, false>(upl);
-  return table ? wave_for_upl<KP_ROPE_INTERLEAVED, true>(upl) : wave_for_upl<KP_ROPE_INTERLEAVED, false>(upl);
-}
-
-// inv[f] = fp32(theta^(-2f/D)), f < D / 2, as products of 16 + D / 32 powers:
-// each within a couple of fp64 roundings, far below fp32's.
-void fill_inv_freq(double theta, int64_t D, float* inv) {
-  double lo[16];
-  for (int i = 0; i < 16; ++i) lo[i] = pow(theta, -(double)(2 * i) / (double)D);
-  double hi = 1.0;
-  for (int f = 0; f < (int)(D / 2); ++f) {
-    if ((f & 15) == 0) hi = pow(theta, -(double)(2 * f) / (double)D);
-    inv[f] = (float)(hi * lo[f & 15]);
-  }
+  const int entries = inv_entries(table, a.D);
+  return half ? wave_kernel<KP_ROPE_HALF>(upl, entries) : wave_kernel<KP_ROPE_INTERLEAVED>(upl, entries);
 }
 
 bool tensor_vec_ok(const RopeTensor& t, int64_t D, int pairing) {
@@ -894,7 +895,10 @@ static int rope_impl(const char* who, const void* x0, void* out0, int64_t H0, co
   a.frs = freq_row_stride;
   a.conj = conj ? 1 : 0;
   a.err = error_flag;
-  if (freqs_cis == nullptr) fill_inv_freq(theta, D, a.inv_freq);
+  float inv[kMaxHalf];  // the InvFreq argument: as many entries of it as the kernel takes
+  const int entries = inv_entries(freqs_cis != nullptr, D);
+  if (freqs_cis == nullptr) fill_inv_freq(theta, (int)D, inv);
+  for (int f = freqs_cis == nullptr ? (int)(D / 2) : 0; f < entries; ++f) inv[f] = 0.f;
   const int64_t npos = B * S;
   if (npos == 0) return KP_OK;
 
@@ -919,7 +923,7 @@ static int rope_impl(const char* who, const void* x0, void* out0, int64_t H0, co
     ta.frs = a.frs;
     ta.conj = a.conj;
     ta.err = a.err;
-    for (int f = 0; f < 64; ++f) ta.inv_freq[f] = a.inv_freq[f];
+    for (int f = 0; f < entries; ++f) ta.inv_freq[f] = inv[f];
     const bool tab = freqs_cis != nullptr, half = pairing == KP_ROPE_HALF;
     const void* fk = half ? (tab ? reinterpret_cast<const void*>(rope_tile<KP_ROPE_HALF, true>)
                                  : reinterpret_cast<const void*>(rope_tile<KP_ROPE_HALF, false>))
@@ -938,28 +942,31 @@ static int rope_impl(const char* who, const void* x0, void* out0, int64_t H0, co
       a.t[0].out = out0_copy;
       if (a.nt > 1) a.t[1].out = out1_copy;
     }
-    const RopeKernel fk = vec ? pick_fast(a, pairing, freqs_cis != nullptr) : nullptr;
+    const void* fk = vec ? pick_fast(a, pairing, freqs_cis != nullptr) : nullptr;
     const bool tab = freqs_cis != nullptr;
     hipStream_t st_ = as_stream(stream);
     Div32 by_c{}, by_s{};
     uint32_t step = 0;
-    const WaveKernel wk = fk == nullptr ? pick_wave(a, pairing, tab, &by_c, &by_s, &step) : nullptr;
+    const void* wk = fk == nullptr ? pick_wave(a, pairing, tab, &by_c, &by_s, &step) : nullptr;
     if (fk != nullptr && blocks_needed <= INT32_MAX) {
-      void* args[] = {&a};
-      launch_dominant_raw(reinterpret_cast<const void*>(fk), dim3((unsigned)blocks_needed), dim3(kThreads), args, 0, st_);
+      void* args[] = {&a, inv};
+      launch_dominant_raw(fk, dim3((unsigned)blocks_needed), dim3(kThreads), args, 0, st_);
     } else if (wk != nullptr) {
       // a position per wave: as many launches as it takes blocks
       for (int64_t b0 = 0; b0 < blocks_needed; b0 += max_blocks(kThreads)) {
         const int64_t nb = blocks_needed - b0 < max_blocks(kThreads) ? blocks_needed - b0 : max_blocks(kThreads);
         uint32_t first = (uint32_t)(b0 * kWavesPerBlock);
-        void* args[] = {&a, &by_c, &by_s, &step, &first};
-        launch_dominant_raw(reinterpret_cast<const void*>(wk), dim3((unsigned)nb), dim3(kThreads), args, 0, st_);
+        void* args[] = {&a, &by_c, &by_s, &step, &first, inv};
+        launch_dominant_raw(wk, dim3((unsigned)nb), dim3(kThreads), args, 0, st_);
       }
     } else {
       const int64_t cap = (int64_t)cu_count() * 16;
       const int grid = (int)(blocks_needed < cap ? blocks_needed : cap);
-      if (tab) KP_LAUNCH_DOMINANT(rope_scalar<true>, dim3(grid), dim3(kThreads), 0, st_, a);
-      else KP_LAUNCH_DOMINANT(rope_scalar<false>, dim3(grid), dim3(kThreads), 0, st_, a);
+      for (int f = entries; f < kMaxHalf; ++f) inv[f] = 0.f;  // rope_scalar takes them all
+      void* args[] = {&a, inv};
+      launch_dominant_raw(tab ? reinterpret_cast<const void*>(rope_scalar<true>)
+                              : reinterpret_cast<const void*>(rope_scalar<false>),
+                          dim3(grid), dim3(kThreads), args, 0, st_);
     }
     const int st = check_launch(who);
     if (st != KP_OK) return st;
