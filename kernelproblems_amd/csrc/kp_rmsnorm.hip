@@ -251,7 +251,7 @@ bool pick_fwd(int64_t M, int64_t N, int* vpl, int* wpr) {
 // 3.1 -> 2.6, 8192 3.5 -> 3.1; 256 rows of 4096 5.1 -> 3.7, 1024 rows 7.1
 // both).  The forward and the gathered forward share the rule, so that a
 // gathered row has the bits of the same row given directly.
-bool few_wide_rows(int64_t M, int64_t N) { return N > 2048 && M <= cu_count(); }
+bool few_wide_rows(int64_t M, int64_t N, int cus) { return N > 2048 && M <= cus; }
 
 // Backward row shape: N = 8192 runs 8 waves per row with 2 chunks per lane in
 // 8-wave blocks (one row per block step; measured on MI355X at [16384, 8192]
@@ -415,11 +415,12 @@ int rms_fwd_impl(const char* who, const void* const* x_terms, const int64_t* x_s
   a.N = N;
   a.eps = eps;
 
+  const int cus = cu_count();  // once: it asks the runtime for the current device
   int vpl = 0, wpr = 0;
   bool vec = pick_fwd(M, N, &vpl, &wpr) && rows_vec_ok(x_terms, x_strides, n_x) && aligned16(y) && (y_stride & 7) == 0;
   if (vec && h_out) vec = aligned16(h_out) && (h_stride & 7) == 0;
   if (vec && weight) vec = aligned16(weight) && (w_seg_len & 7) == 0 && (w_seg_stride & 7) == 0;
-  vec = vec && !(few_rows && few_wide_rows(M, N));
+  vec = vec && !(few_rows && few_wide_rows(M, N, cus));
   const FwdKernel fk = vec ? fwd_kernel(vpl, wpr, n_x) : nullptr;
   vec = vec && fk != nullptr;
   hipStream_t s = as_stream(stream);
@@ -431,7 +432,7 @@ int rms_fwd_impl(const char* who, const void* const* x_terms, const int64_t* x_s
     // against 185 us for 2 pipelined blocks per CU.  Shorter rows (1 or 2
     // waves) keep the pipelined grid ([4096, 4096]: 12.5 us against 13.8 us
     // for one block per 4 rows).
-    const int64_t cap = wpr == 4 ? groups : (int64_t)cu_count() * fwd_bpc((int64_t)n_x * vpl * 1024);
+    const int64_t cap = wpr == 4 ? groups : (int64_t)cus * fwd_bpc((int64_t)n_x * vpl * 1024);
     if (groups > INT32_MAX) return fail(KP_EUNSUPPORTED, "%s: too many rows for one launch", who);
     const int grid = (int)(groups < cap ? groups : cap);
     void* args[] = {&a};
@@ -446,12 +447,12 @@ int rms_fwd_impl(const char* who, const void* const* x_terms, const int64_t* x_s
   // so are rows on 16-byte addresses once the call's traffic is beyond the
   // Infinity Cache ([8192, 5120] two terms 56.0 / 58.9).
   AnyShape as{}, ls{};
-  const FwdKernel ak = any_fwd_shape(M * n_x, N, cu_count(), &as) ? fwd_any_kernel(as, n_x) : nullptr;
+  const FwdKernel ak = any_fwd_shape(M * n_x, N, cus, &as) ? fwd_any_kernel(as, n_x) : nullptr;
   const bool streamed = (N & 7) == 0 && rows_vec_ok(x_terms, x_strides, n_x) &&
                         M * N * 2 * (n_x + (n_x > 1 && h_out != nullptr ? 2 : 1)) > ((int64_t)160 << 20);
-  const FwdKernel lk = M > cu_count() && !streamed && any_loop_shape(N, &ls) ? fwd_any_loop_kernel(ls, n_x) : nullptr;
+  const FwdKernel lk = M > cus && !streamed && any_loop_shape(N, &ls) ? fwd_any_loop_kernel(ls, n_x) : nullptr;
   if (lk != nullptr) {
-    const int64_t lgroups = ceil_div(M, 4 / ls.wpr), cap = (int64_t)cu_count() * fwd_bpc((int64_t)n_x * ls.vpl * 1024);
+    const int64_t lgroups = ceil_div(M, 4 / ls.wpr), cap = (int64_t)cus * fwd_bpc((int64_t)n_x * ls.vpl * 1024);
     void* args[] = {&a};
     launch_dominant_raw(reinterpret_cast<const void*>(lk), dim3((unsigned)(lgroups < cap ? lgroups : cap)),
                         dim3(kThreads), args, 0, s);
@@ -462,7 +463,7 @@ int rms_fwd_impl(const char* who, const void* const* x_terms, const int64_t* x_s
     void* args[] = {&a};
     launch_dominant_raw(reinterpret_cast<const void*>(ak), dim3((unsigned)groups), dim3(kThreads), args, 0, s);
   } else {
-    const int64_t cap = (int64_t)cu_count() * 8;
+    const int64_t cap = (int64_t)cus * 8;
     const int grid = (int)(M < cap ? M : cap);
     KP_LAUNCH_DOMINANT(rms_fwd_generic, dim3(grid), dim3(kThreads), 0, s, a);
   }
@@ -685,6 +686,7 @@ int kp_embedding_rmsnorm_fwd_bf16(const void* table, int64_t V, int64_t table_ro
   a.N = N;
   a.eps = eps;
 
+  const int cus = cu_count();
   int vpl = 0, wpr = 0;
   // one wave per row beyond a few (few_wide_rows): the gather's row-per-block
   // form measured 39.3 against 34.2 us at C3 (cache-served table rows favour
@@ -697,7 +699,7 @@ int kp_embedding_rmsnorm_fwd_bf16(const void* table, int64_t V, int64_t table_ro
   if (fk == nullptr)
     return fail(KP_EUNSUPPORTED, "%s: row shape / alignment without a fused kernel (N=%lld)", who, (long long)N);
   AnyShape as{};
-  if (few_wide_rows(T, N) && any_fwd_shape(T, N, cu_count(), &as)) {
+  if (few_wide_rows(T, N, cus) && any_fwd_shape(T, N, cus, &as)) {
     if (const FwdKernel ak = fwd_any_gather_kernel(as)) {
       void* args[] = {&a};
       launch_dominant_raw(reinterpret_cast<const void*>(ak), dim3((unsigned)T), dim3(kThreads), args, 0,
@@ -708,7 +710,7 @@ int kp_embedding_rmsnorm_fwd_bf16(const void* table, int64_t V, int64_t table_ro
   const int rb = 4 / wpr;
   const int64_t groups = ceil_div(T, rb);
   // one block per row for rows of 4 waves, as in kp_rmsnorm_fwd_bf16
-  const int64_t cap = wpr == 4 ? groups : (int64_t)cu_count() * fwd_bpc((int64_t)vpl * 1024);
+  const int64_t cap = wpr == 4 ? groups : (int64_t)cus * fwd_bpc((int64_t)vpl * 1024);
   if (groups > INT32_MAX) return fail(KP_EUNSUPPORTED, "%s: too many rows for one launch", who);
   const int grid = (int)(groups < cap ? groups : cap);
   void* args[] = {&a};
