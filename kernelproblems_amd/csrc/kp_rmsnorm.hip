@@ -443,13 +443,17 @@ int rms_fwd_impl(const char* who, const void* const* x_terms, const int64_t* x_s
   // run the persistent loop (us, one-shot / loop: [3001, 2880] two terms 14.0 /
   // 12.3, [4096, 4095] 15.8 / 13.8, [16384, 2881] two terms 79.8 / 72.5); few
   // or short rows are as fast or faster with a block each ([2048, 1001] two
-  // terms 4.9 / 5.2), wider ones too ([8192, 5121] two terms 72.0 / 74.9), and
-  // so are rows on 16-byte addresses once the call's traffic is beyond the
-  // Infinity Cache ([8192, 5120] two terms 56.0 / 58.9).
+  // terms 4.9 / 5.2), wider ones too ([8192, 5121] two terms 72.0 / 74.9).
+  // So are rows on 16-byte addresses once the call moves more than about 100
+  // MiB: over widths from 1032 to 5112 the loop takes 0.85 to 1.04 of the
+  // one-shot time at 40 MiB and 0.94 to 1.08 at 80, then the one-shot form is
+  // ahead (two terms: [12211, 1288], 120 MiB, 24.3 / 25.9; [4388, 3584] 23.2 /
+  // 24.5; [10922, 2880], 240 MiB, 42.3 / 46.8; [13653, 4608], 480 MiB, 82.3 /
+  // 92.3; [121927, 1032], 960 MiB, 179 / 230).
   AnyShape as{}, ls{};
   const FwdKernel ak = any_fwd_shape(M * n_x, N, cus, &as) ? fwd_any_kernel(as, n_x) : nullptr;
   const bool streamed = (N & 7) == 0 && rows_vec_ok(x_terms, x_strides, n_x) &&
-                        M * N * 2 * (n_x + (n_x > 1 && h_out != nullptr ? 2 : 1)) > ((int64_t)160 << 20);
+                        M * N * 2 * (n_x + (n_x > 1 && h_out != nullptr ? 2 : 1)) > ((int64_t)100 << 20);
   const FwdKernel lk = M > cus && !streamed && any_loop_shape(N, &ls) ? fwd_any_loop_kernel(ls, n_x) : nullptr;
   if (lk != nullptr) {
     const int64_t lgroups = ceil_div(M, 4 / ls.wpr), cap = (int64_t)cus * fwd_bpc((int64_t)n_x * ls.vpl * 1024);

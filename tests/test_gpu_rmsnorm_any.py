@@ -63,9 +63,10 @@ def test_widths(gpu, N, M, terms):
 
 
 @pytest.mark.parametrize("M,N", [(131077, 33), (131077, 64), (66001, 128), (33000, 200), (17001, 500), (9001, 1000),
-                                 (40000, 2049), (20000, 4098)])
+                                 (40000, 2049), (20000, 4098), (20000, 2056), (12000, 4104)])
 def test_many_rows(gpu, M, N):
-    """Enough rows for several per lane group, and traffic beyond the persistent loop's."""
+    """Enough rows for several per lane group; long walks of the persistent loop (odd widths), and the one-shot form
+    that 16-byte rows take instead beyond its traffic (2056 and 4104 columns)."""
     x = [_rand(gpu, i, M, N) for i in range(2)]
     w = _rand(gpu, 7, N) * 0.02 + 1
     h, y, rstd = kp.rms_norm(x, w, EPS, N, return_h=True)
