@@ -1099,7 +1099,7 @@ bool ranked_in_sort(const EmbBwdArgs& a) { return a.nchunks == 1 && a.V <= kRank
 int launch_sort(const char* who, const EmbBwdArgs& a, const ZeroShares& Z, bool first, hipStream_t s) {
   const int64_t rank_blocks = ceil_div((int64_t)a.nchunks * kChunk, kThreads);
   const int64_t g1 = a.nchunks + ceil_div(Z.s1.units, kSortThreads), g2 = rank_blocks + zero_blocks(Z.s2);
-  if (g1 > 0x7fffffffLL || g2 > 0x7fffffffLL) return fail(KP_EUNSUPPORTED, "%s: V * D too large for one launch", who);
+  if (g1 > max_blocks(kSortThreads) || g2 > max_blocks(kThreads)) return fail(KP_EUNSUPPORTED, "%s: V * D too large for one launch", who);
   if (ranked_in_sort(a)) {
     KP_LAUNCH_SPAN(first, false, emb_sort_chunks<true>, dim3((unsigned)g1), dim3(kSortThreads),
                    (size_t)ceil_div(a.V, 32) * 4, s, a, Z.s1);
@@ -1228,7 +1228,7 @@ int kp_embedding_bwd_bf16(const void* grad, int64_t grad_row_stride, const void*
     a.out = static_cast<uint8_t*>(grad_table) + lo * row_bytes;
     const ZeroShares Z = make_shares(Vs, row_bytes, ranked_in_sort(a), combine);
     const int64_t g3 = nwin_blocks + zero_blocks(Z.s3), g4 = comb_blocks + zero_blocks(Z.s4);
-    if (g3 > 0x7fffffffLL || g4 > 0x7fffffffLL)
+    if (g3 > max_blocks(kThreads) || g4 > max_blocks(kThreads))
       return fail(KP_EUNSUPPORTED, "%s: V * D too large for one launch", who);
     // With the timing hook set, the events span the whole pipeline (the first
     // launch's start to the last one's end): its zero fill is spread over them.
@@ -1364,7 +1364,7 @@ int kp_rmsnorm_embedding_bwd_bf16(const void* const* dy_terms, const int64_t* dy
   const ZeroShares Z = make_shares(V, row_bytes, ranked_in_sort(e), true);
   const int comb_blocks = (int)(L.nwin * nq < cu_count() * 4 ? L.nwin * nq : cu_count() * 4);
   const int64_t g3 = zero_blocks(Z.s3), g4 = comb_blocks + zero_blocks(Z.s4);
-  if (g3 > 0x7fffffffLL || g4 > 0x7fffffffLL)
+  if (g3 > max_blocks(kThreads) || g4 > max_blocks(kThreads))
     return fail(KP_EUNSUPPORTED, "%s: V * N too large for one launch", who);
   int st = launch_sort(who, e, Z, true, s);
   if (st != KP_OK) return st;

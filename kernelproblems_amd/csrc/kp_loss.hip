@@ -799,11 +799,22 @@ int kp_cross_entropy_fwd_bf16(const void* logits, int64_t row_stride, int64_t M,
                      : nt == 64  ? reinterpret_cast<const void*>(xent_fwd_vec<64>)
                      : nt == 256 ? reinterpret_cast<const void*>(xent_fwd_vec<256>)
                                  : reinterpret_cast<const void*>(xent_fwd_vec<1024>);
-    const unsigned blocks = (unsigned)(nt > 64 ? M : ceil_div(M, kWavesPerBlock));
-    void* args[] = {&a};
-    launch_dominant_raw(fk, dim3(blocks), dim3(nt > kThreads ? nt : kThreads), args, 0, st);
-    const int rc = check_launch(who);
-    if (rc != KP_OK) return rc;
+    // Rows in slabs of what one launch takes (several only at a wave per row).
+    constexpr int64_t kSlab = max_blocks(kThreads) * kWavesPerBlock;
+    for (int64_t r0 = 0; r0 < M; r0 += kSlab) {
+      FwdArgs b = a;
+      b.M = M - r0 < kSlab ? M - r0 : kSlab;
+      b.logits += r0 * row_stride;
+      b.targets = static_cast<const char*>(targets) + r0 * target_bytes;
+      b.row_loss += r0;
+      b.row_valid += r0;
+      if (row_lse != nullptr) b.lse_out += r0;
+      const unsigned blocks = (unsigned)(nt > 64 ? b.M : ceil_div(b.M, kWavesPerBlock));
+      void* args[] = {&b};
+      launch_dominant_raw(fk, dim3(blocks), dim3(nt > kThreads ? nt : kThreads), args, 0, st);
+      const int rc = check_launch(who);
+      if (rc != KP_OK) return rc;
+    }
   }
   hipLaunchKernelGGL(xent_fwd_finish, dim3(1), dim3(kFinThreads), 0, st, a.row_loss, a.row_valid, M, (double)scale,
                      loss, total_weight);
@@ -836,9 +847,8 @@ int kp_cross_entropy_bwd_bf16(const float* log_softmax, int64_t lsm_row_stride, 
   const bool vec = V % 4 == 0 && aligned16(log_softmax) && (reinterpret_cast<uintptr_t>(grad_logits) & 7) == 0 &&
                    (M == 1 || (lsm_row_stride % 4 == 0 && out_row_stride % 4 == 0));
   void* args[] = {&a};
-  if (vec) {
-    const int64_t bpr = ceil_div(V / 4, kBwdBlockGroups);
-    if (bpr * M > 0x7fffffffLL) return fail(KP_EUNSUPPORTED, "%s: too many blocks", who);
+  const int64_t bpr = ceil_div(V, 4 * kBwdBlockGroups);  // blocks per row
+  if (vec && bpr <= max_blocks(kThreads) / M) {
     a.bpr = (int)bpr;
     launch_dominant_raw(reinterpret_cast<const void*>(xent_bwd_vec), dim3((unsigned)(bpr * M)), dim3(kThreads), args,
                         0, as_stream(stream));

@@ -432,7 +432,7 @@ int rms_fwd_impl(const char* who, const void* const* x_terms, const int64_t* x_s
     // against 185 us for 2 pipelined blocks per CU.  Shorter rows (1 or 2
     // waves) keep the pipelined grid ([4096, 4096]: 12.5 us against 13.8 us
     // for one block per 4 rows).
-    const int64_t cap = wpr == 4 ? groups : (int64_t)cus * fwd_bpc((int64_t)n_x * vpl * 1024);
+    const int64_t cap = wpr == 4 ? max_blocks(kThreads) : (int64_t)cus * fwd_bpc((int64_t)n_x * vpl * 1024);
     if (groups > INT32_MAX) return fail(KP_EUNSUPPORTED, "%s: too many rows for one launch", who);
     const int grid = (int)(groups < cap ? groups : cap);
     void* args[] = {&a};
@@ -714,7 +714,7 @@ int kp_embedding_rmsnorm_fwd_bf16(const void* table, int64_t V, int64_t table_ro
   const int rb = 4 / wpr;
   const int64_t groups = ceil_div(T, rb);
   // one block per row for rows of 4 waves, as in kp_rmsnorm_fwd_bf16
-  const int64_t cap = wpr == 4 ? groups : (int64_t)cus * fwd_bpc((int64_t)vpl * 1024);
+  const int64_t cap = wpr == 4 ? max_blocks(kThreads) : (int64_t)cus * fwd_bpc((int64_t)vpl * 1024);
   if (groups > INT32_MAX) return fail(KP_EUNSUPPORTED, "%s: too many rows for one launch", who);
   const int grid = (int)(groups < cap ? groups : cap);
   void* args[] = {&a};

@@ -942,13 +942,15 @@ static int rope_impl(const char* who, const void* x0, void* out0, int64_t H0, co
       a.t[0].out = out0_copy;
       if (a.nt > 1) a.t[1].out = out1_copy;
     }
-    const void* fk = vec ? pick_fast(a, pairing, freqs_cis != nullptr) : nullptr;
+    // rope_fast takes a position per wave in one launch, rope_wave in several
+    const void* fk =
+        vec && blocks_needed <= max_blocks(kThreads) ? pick_fast(a, pairing, freqs_cis != nullptr) : nullptr;
     const bool tab = freqs_cis != nullptr;
     hipStream_t st_ = as_stream(stream);
     Div32 by_c{}, by_s{};
     uint32_t step = 0;
     const void* wk = fk == nullptr ? pick_wave(a, pairing, tab, &by_c, &by_s, &step) : nullptr;
-    if (fk != nullptr && blocks_needed <= INT32_MAX) {
+    if (fk != nullptr) {
       void* args[] = {&a, inv};
       launch_dominant_raw(fk, dim3((unsigned)blocks_needed), dim3(kThreads), args, 0, st_);
     } else if (wk != nullptr) {
