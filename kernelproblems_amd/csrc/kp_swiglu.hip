@@ -282,7 +282,20 @@ int launch_pointwise(const char* who, int op, const void* const* in, const int64
   for (int i = 0; i < nin; ++i) flat = flat && (M == 1 || in_rs[i] == N);
   for (int i = 0; i < nout; ++i) flat = flat && (M == 1 || out_rs[i] == N);
   const int64_t n = flat ? M * N : N, rows = flat ? 1 : M, cpr = ceil_div(n, 8);
-  if (n >= 8 && (flat || cpr <= kMaxRowChunks / rows)) {
+  if (n >= 8 && !flat && cpr > kMaxRowChunks / rows) {
+    // More chunks than one launch numbers (34 GB an array): rows in slabs.
+    const int64_t slab = cpr < kMaxRowChunks ? kMaxRowChunks / cpr : 1;
+    for (int64_t r0 = 0; r0 < M; r0 += slab) {
+      const void* sin[4];
+      void* sout[3];
+      for (int i = 0; i < nin; ++i) sin[i] = static_cast<const uint16_t*>(in[i]) + r0 * in_rs[i];
+      for (int i = 0; i < nout; ++i) sout[i] = static_cast<uint16_t*>(out[i]) + r0 * out_rs[i];
+      const int st = launch_pointwise(who, op, sin, in_rs, sout, out_rs, M - r0 < slab ? M - r0 : slab, N, stream);
+      if (st != KP_OK) return st;
+    }
+    return KP_OK;
+  }
+  if (n >= 8) {
     VecArgs a{};
     for (int i = 0; i < nin; ++i) {
       a.in[i] = static_cast<const uint16_t*>(in[i]);
