@@ -55,7 +55,7 @@ struct RopeArgs {
 // identical).  A kernel's last argument, of no more entries than it needs
 // (none in table mode, 64 for D <= 128): a call of few positions is bound by
 // its host time.  16 tokens of 32 + 8 heads of 64 from theta: 5.65 us with all
-// 256 in every call's arguments and 16 + D / 32 powers, 5.45 us so.
+// 256 in every call's arguments and 16 + D / 32 powers, 5.4 us so.
 template <int F>
 struct InvFreq {
   float f[F];

@@ -18,7 +18,7 @@ int main() {
         const long double unit = ldexpl(1.0L, ilogbl(exact) - 23);
         ++checked;
         differ += inv[f] != want;
-        if (fabsl((long double)inv[f] - exact) > unit * (0.5L + 0x1p-22L)) {
+        if (fabsl((long double)inv[f] - exact) > unit * (0.5L + 0x1p-23L)) {
           ++bad;
           std::printf("theta %g D %d f %d: %.9g, exact %.12Lg\n", theta, D, f, inv[f], exact);
         }
