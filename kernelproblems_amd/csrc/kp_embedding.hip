@@ -686,6 +686,35 @@ __global__ __launch_bounds__(kThreads) void emb_dense(EmbBwdArgs a, int64_t n_wi
   zero_block(a, z, b - n_win_blocks);
 }
 
+// K3 of the chain, whose windows are the fused row pass: the conditional share
+// alone, over rows of whole 16-byte units (the chain's are multiples of 512
+// columns).  Bound by HBM writes, whose rate falls with more blocks than it
+// needs in flight, so the launch asks for LDS that it does not use: blocks per
+// CU 8 (none), 7, 6, 5, 4, 3 take the chain of [8192, 4096] into an fp32
+// [128256, 4096] table 401, 396.7, 388.6, 381.3, 381.3, 471 us.  As window-less
+// blocks of emb_dense (7 per CU by its registers, and a chain of scalar loads
+// ahead of a block's store) 390.0, and 387.5 before rows of any width.
+constexpr size_t kZeroRowsLds = 32 * 1024;  // 5 blocks per CU of 160 KiB
+struct ZeroRows {
+  char* out;             // the share's first row
+  const uint32_t* bits;  // touched rows
+  uint32_t lo, hi, units;
+  Div32 upr;  // units per row
+};
+__global__ __launch_bounds__(kThreads) void emb_zero_rows(ZeroRows z) {
+  const uint32_t u0 = blockIdx.x * kThreads, u = u0 + threadIdx.x;
+  uint32_t r = div32(u0, z.upr);
+  if (u0 + kThreads <= (r + 1) * z.upr.d) {  // the whole block in one row: one scalar test
+    r += z.lo;
+    if (r >= z.hi || ((z.bits[r >> 5] >> (r & 31)) & 1u) != 0) return;
+  } else {
+    if (u >= z.units) return;
+    r = div32(u, z.upr) + z.lo;
+    if (((z.bits[r >> 5] >> (r & 31)) & 1u) != 0) return;
+  }
+  st16u_stream(reinterpret_cast<uint16_t*>(z.out + (uint64_t)u0 * 16 + threadIdx.x * 16), u32x4{0u, 0u, 0u, 0u});
+}
+
 // ---- K4: runs spanning windows, pieces added in window order ---------------
 // Blocks [0, comb_blocks) walk the windows grid-stride; later blocks are the
 // launch's (conditional) zero share.
@@ -1374,7 +1403,13 @@ int kp_rmsnorm_embedding_bwd_bf16(const void* const* dy_terms, const int64_t* dy
     if ((st = check_launch(who)) != KP_OK) return st;
   }
   if (g3 > 0) {
-    hipLaunchKernelGGL(emb_dense<true>, dim3((unsigned)g3), dim3(kThreads), 0, s, e, (int64_t)0, Z.s3);
+    if (Z.s3.rep == 1) {
+      const ZeroRows z{static_cast<char*>(grad_table) + Z.s3.lo * row_bytes, e.bitmap, (uint32_t)Z.s3.lo,
+                       (uint32_t)Z.s3.hi, (uint32_t)Z.s3.units, Z.s3.upr};
+      hipLaunchKernelGGL(emb_zero_rows, dim3((unsigned)g3), dim3(kThreads), kZeroRowsLds, s, z);
+    } else {
+      hipLaunchKernelGGL(emb_dense<true>, dim3((unsigned)g3), dim3(kThreads), 0, s, e, (int64_t)0, Z.s3);
+    }
     if ((st = check_launch(who)) != KP_OK) return st;
   }
   if (g4 > 0) KP_LAUNCH_SPAN(false, true, emb_combine<true>, dim3((unsigned)g4), dim3(kThreads), 0, s, e, comb_blocks, Z.s4);
