@@ -97,6 +97,13 @@ void kp_debug_block_trace(void* buf, size_t bytes);
  *   (a contiguous weight has w_seg_len = N); NULL means no weight.
  * y (bf16 [M, N], row stride y_stride) = bf16(fp32(h) * rstd * fp32(w)).
  * rstd (fp32 [M], may be NULL) = 1 / sqrt(sum(h^2) / N + eps).
+ *
+ * The order in which a row's squares are summed depends on N, on the
+ * alignment and, for some N, on M: up to the CU count and beyond it (N from
+ * 1025 to 5120, and multiples of 512 above 2048), from 8192 rows on (N =
+ * 4096), and past 100 MiB of traffic (16-byte rows of 1025 to 5120 columns
+ * whose N is no multiple of 512, or 3584 or 4608).  So the same row may get an
+ * rstd and y that differ in their last bit from a call of another M.
  */
 int kp_rmsnorm_fwd_bf16(const void* const* x_terms, const int64_t* x_strides, int n_x,
                         const void* weight, int64_t w_seg_len, int64_t w_seg_stride,
@@ -191,7 +198,9 @@ int kp_rmsnorm_bwd_bf16_noalloc(const void* const* dy_terms, const int64_t* dy_s
  *   y (bf16 [M, N], row stride y_stride) = bf16(fp32(x) * rstd * fp32(w)),
  *   h_out (bf16 [M, N], may be NULL) = the summed x terms when n_x > 1,
  *   rstd_out (fp32 [M], may be NULL) = the rstd both halves used,
- * reading x once where the two-operator sequence reads it twice.
+ * reading x once where the two-operator sequence reads it twice.  Widths,
+ * alignments and term counts without a one-pass kernel run the forward and
+ * then the backward with the forward's rstd.
  * workspace: at least kp_rmsnorm_fwd_bwd_workspace_size(M, N) bytes, 16-byte aligned.
  */
 size_t kp_rmsnorm_fwd_bwd_workspace_size(int64_t M, int64_t N);
@@ -225,7 +234,9 @@ int kp_rmsnorm_fwd_bwd_bf16(const void* const* dy_terms, const int64_t* dy_strid
  * error_flag != NULL, *error_flag is set to 1.
  * Rows, strides and pointers must be 16-byte granular with N a fast-path row
  * length; otherwise KP_EUNSUPPORTED (compose kp_embedding_fwd_bf16 and
- * kp_rmsnorm_fwd_bf16 instead).
+ * kp_rmsnorm_fwd_bf16 instead).  h, y and rstd are bit for bit those of that
+ * composition, except that from 8192 rows of N = 4096 on rstd and y may differ
+ * in their last bit.
  */
 int kp_embedding_rmsnorm_fwd_bf16(const void* table, int64_t V, int64_t table_row_stride, const void* indices,
                                   int index_bytes, int64_t T, const void* weight, int64_t w_seg_len,
@@ -560,12 +571,15 @@ int kp_cross_entropy_bwd_bf16(const float* log_softmax, int64_t lsm_row_stride, 
  * forward's (kp_cross_entropy_fwd_bf16).  logits / grad_logits: bf16 [M, V],
  * unit inner stride, row strides in elements; grad_logits may be logits
  * itself (in place).  Rows with an ignored or out-of-range target get zero
- * gradient (out-of-range ones also set *error_flag).  loss and total_weight
+ * gradient (out-of-range ones also set *error_flag).  A row that holds NaN or
+ * +inf, or -inf alone, gets NaN in every column whatever its target, as the
+ * exp of its NaN log-softmax gives in eager.  loss and total_weight
  * are both NULL (no forward outputs, no workspace) or both given; then the
  * workspace is kp_cross_entropy_fwd_workspace_size(M) bytes, 8-byte aligned.
- * One launch holds each row in registers when V % 8 == 0, V <= 131072 and
- * rows are 16-byte aligned (4 bytes of HBM traffic per element); other
- * shapes take two passes over the row.
+ * One launch holds each row in registers for 8 <= V <= 131072, any row stride
+ * and alignment (4 bytes of HBM traffic per element; rows off a 16-byte
+ * boundary take about 1.17 times as long); other V take two passes over the
+ * row.
  */
 int kp_cross_entropy_fwd_bwd_bf16(const void* logits, int64_t row_stride, int64_t M, int64_t V,
                                   const void* targets, int target_bytes, int64_t ignore_index,

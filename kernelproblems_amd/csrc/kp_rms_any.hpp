@@ -24,7 +24,7 @@
 // twice, the weight-gradient partials updated in memory):
 //   add + norm forward [3001, 2880]        35.9 -> 12.3 us (5.6 TB/s)
 //   forward + backward [65536, 128]       275   -> 19.7 us (two row kernels and the finalize, 84 MB)
-//   forward + backward of odd widths      8.9x at 90 us
+//   backward of [2048, 11001]             338   -> 44.9 us
 #pragma once
 
 #include "kp_rms_shapes.hpp"
@@ -270,6 +270,11 @@ __global__ __launch_bounds__(kThreads) void rms_fwd_any_loop(RmsFwdArgs a) {
 // rms_bwd_vec).  The column sums of the block's rows stay in registers; at
 // the end its 8 / WPR x 64 / LPR row slots are added per column in slot order
 // through LDS and written as one partial row, in rms_dw_finalize's layout.
+// Rows of 12289 columns and more hold 4 chunks per lane: past 256 VGPRs with a
+// second term or a residual, where the compiler spills 6 to 95 of them to
+// scratch (a residual and three terms of 8193 to 12288 columns: 4).  They
+// stay 6.6 to 11 times faster than the scalar kernel even so ([2048, 16384],
+// one term 501 -> 50.6 us, two and two with a residual 1088 -> 128.5).
 template <int VPL, int NX, int NDY, bool RES>
 struct AnySlot {
   u32x4 x[NX][VPL], d[NDY][VPL], r[VPL];  // r: the residual gradient (RES)
