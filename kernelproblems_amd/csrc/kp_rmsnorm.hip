@@ -247,9 +247,9 @@ bool pick_fwd(int64_t M, int64_t N, int* vpl, int* wpr) {
 
 // A few wide rows: four waves per row from the kernels for any width, a block
 // per row, finish sooner than a row's one or two waves, and without the large
-// grid's starting pause (two terms, 16 rows: 4096 columns 4.0 -> 2.7 us, 2560
-// 3.1 -> 2.6, 8192 3.5 -> 3.1; 256 rows of 4096 5.1 -> 3.7, 1024 rows 7.1
-// both).  The forward and the gathered forward share the rule, so that a
+// grid's starting pause (kernel medians, two terms, 16 rows: 4096 columns 3.8
+// -> 3.1 us, 8192 3.8 -> 3.6, 2560 3.0 and 3.1; 256 rows of 4096 5.2 -> 4.0,
+// 1024 rows 7.1 both).  The forward and the gathered forward share the rule, so that a
 // gathered row has the bits of the same row given directly.
 bool few_wide_rows(int64_t M, int64_t N, int cus) { return N > 2048 && M <= cus; }
 
